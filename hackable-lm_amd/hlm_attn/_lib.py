@@ -9,7 +9,7 @@ import ctypes
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().with_name("libhlm_attn.so")
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 # Every symbol include/hlm_attn.h declares, with its (restype, argtypes).
 _P = ctypes.c_void_p
@@ -28,6 +28,9 @@ SIGNATURES["hlm_attn_bwd_noalloc"] = (_I, _BWD_ARGTYPES[:9] + _BWD_ARGTYPES[10:]
 # the single-pass backward: + partial workspace (pointer, bytes) after delta_ws
 SIGNATURES["hlm_attn_bwd_fused"] = (_I, _BWD_ARGTYPES[:10] + [_P, ctypes.c_int64] + _BWD_ARGTYPES[10:])
 SIGNATURES["hlm_attn_bwd_fused_workspace_bytes"] = (ctypes.c_int64, [_I, _I, _I, _I, _I])
+# the two-kernel backward with long dK/dV tiles cut into chunks: the same workspace arguments
+SIGNATURES["hlm_attn_bwd_split"] = SIGNATURES["hlm_attn_bwd_fused"]
+SIGNATURES["hlm_attn_bwd_split_workspace_bytes"] = (ctypes.c_int64, [_I, _I, _I, _I, _I, _I])
 SIGNATURES["hlm_attn_fwd_split"] = (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _S, _S, _S, _S, _I, _F, _P])
 SIGNATURES["hlm_attn_fwd_split_count"] = (_I, [_I, _I, _I, _I, _I])
 SIGNATURES["hlm_qk_norm_rope_fwd"] = (_I, [_P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _S, _S, _F, _P])

@@ -6,6 +6,8 @@
 // scheduler, which honours the sched_group_barrier pipeline of the S/dP
 // operand reads below within three waves per SIMD at D = 64; the dQ kernel
 // keeps the iterative-ILP scheduler, which measured 2-5% faster for it.
+#include <algorithm>
+
 #include "attn_common.h"
 
 namespace hlm {
@@ -24,7 +26,7 @@ namespace hlm {
 // as whole rows.  The ring is topped up to NBUF - 1 tiles ahead after each
 // barrier.
 // ---------------------------------------------------------------------------
-template <int D, int NBUF, int PRE>
+template <int D, int NBUF, int PRE, bool SPLIT>
 __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kernel(BwdArgs a) {
   using L = CS<D>;
   constexpr int NW = 4, BNK = NW * 32, BMQ = 32;
@@ -51,7 +53,13 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   const int G = H / Hkv;
   // Rank-major: every kv head's longest key tiles (the low ones) first.
   const TileId tid_ = rank_major(blockIdx.x, a.B * Hkv);
-  const int kt = tid_.rank;
+  int kt = tid_.rank, chunk = 0;
+  if constexpr (SPLIT) {
+    // Ranks run over chunk 0 of every key tile, then chunk 1 of those that
+    // have one, ...
+    while (chunk + 1 < a.split.n && kt >= a.split.base[chunk + 1]) ++chunk;
+    kt -= a.split.base[chunk];
+  }
   const int bhk = tid_.unit;
   const int hk = bhk % Hkv, b = bhk / Hkv;
 
@@ -64,7 +72,9 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   const int q_hi = min(T - 1, k0 + BNK - 1 + W - 1);
   const int tq_lo = q_lo / BMQ, tq_hi = q_hi / BMQ;
   const int nq = tq_hi - tq_lo + 1;
-  const int n_iter = nq * G;
+  // The query tiles this workgroup visits, of the nq * G of its key tile.
+  const int it_lo = SPLIT ? chunk * a.split.len : 0;
+  const int n_iter = SPLIT ? min(a.split.len, nq * G - it_lo) : nq * G;
   const int sq2 = (int)(a.sq[1] * 2), sdo2 = (int)(a.sdo[1] * 2);
 
   // Start values: waves 0 and 2 copy a tile's -lse*log2(e) row, waves 1 and 3
@@ -99,7 +109,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
 
   // 2. Query tiles, visited head by head (the G query heads of this kv head),
   // tile by tile; each copy goes to ring slot (issue index) % NBUF.
-  int ld_g = 0, ld_t = 0, issued = 0, islot = 0;
+  int ld_g = SPLIT ? it_lo / nq : 0, ld_t = SPLIT ? it_lo - ld_g * nq : 0, issued = 0, islot = 0;
+  const int ld_t0 = ld_t;
   // D = 128: query tiles of each head in the rotated order (step t reads the
   // tile congruent to t modulo nq), so that neighbouring key tiles on one XCD
   // stream the same Q and dO rows together: 25-30% fewer L2 misses at W =
@@ -203,7 +214,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
 
   const bool wave_live = kw0 < T;
   const int wk_hi = min(kw0 + 31, T - 1);
-  int cp_t = 0;  // query tile (within the current head) of the compute pointer
+  int cp_t = ld_t0;  // query tile (within the current head) of the compute pointer
 
   // The tile loop is unrolled by the ring depth, so each copy of the body
   // reads a fixed slot: its LDS addresses are a per-lane register (slot 0's
@@ -330,6 +341,30 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
       }
   }
 
+  if constexpr (SPLIT) {
+    if (kt < a.split.base[2] - a.split.base[1]) {
+      // The key tile has more chunks: fp32 partial sums, in the accumulators'
+      // own order ([wave][dK, dV][db][i][lane] x 4 floats, 1 KB a store).
+      // Every issued tile has been waited for inside the loop.
+      f32x4* dst = reinterpret_cast<f32x4*>(a.split.part) +
+                   ((int64_t)(a.split.base[chunk] + kt) * (a.B * Hkv) + bhk) * (BNK * D / 2) + wave * (2 * NDB * 4 * 64) + lane;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f32x4 k4, v4;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            k4[j] = dkacc[db][4 * i + j];
+            v4[j] = dvacc[db][4 * i + j];
+          }
+          dst[(db * 4 + i) * 64] = k4;
+          dst[((NDB + db) * 4 + i) * 64] = v4;
+        }
+      return;
+    }
+  }
+
   // dK and dV through LDS: every wave is past its last tile, so wave w may use
   // the bytes [64 rows * w, 64 rows * (w + 1)) of the ring for its two blocks.
   dma_barrier<0>();
@@ -366,18 +401,122 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   }
 }
 
+// Sums the chunks of a split dK/dV in their order and writes bf16 rows;
+// bound by reading the partial sums once, fully coalesced.  One
+// workgroup per 32 keys of one (batch, kv head) and one of dK, dV: thread
+// (lane, wave) adds the f32x4 pieces piece = wave, wave + 4, ... of the
+// block, and the rows leave through LDS.
+template <int D>
+__global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_merge_kernel(BwdArgs a) {
+  using L = CS<D>;
+  constexpr int NDB = D / 32, PIECES = NDB * 4, PPT = PIECES / 4;  // f32x4 per thread and chunk
+  constexpr int64_t BLOCK = 128 * D / 2;                          // f32x4 per chunk block (dK and dV)
+  __shared__ __attribute__((aligned(1024))) char rows[32 * D * 2];
+  const int units = a.B * a.Hkv, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int which = blockIdx.x & 1, quarter = (blockIdx.x >> 1) & 3;
+  const int kt = (int)(blockIdx.x >> 3) / units, unit = (int)(blockIdx.x >> 3) % units;
+  int n = 0;  // chunks of this key tile
+  while (n < a.split.n && kt < a.split.base[n + 1] - a.split.base[n]) ++n;
+  f32x4 acc[PPT];
+#pragma unroll
+  for (int p = 0; p < PPT; ++p) acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const f32x4* src = reinterpret_cast<const f32x4*>(a.split.part) + quarter * (2 * PIECES * 64) + which * (PIECES * 64) +
+                     wave * 64 + lane;
+  for (int c = 0; c < n; ++c) {
+    const f32x4* s = src + ((int64_t)(a.split.base[c] + kt) * units + unit) * BLOCK;
+#pragma unroll
+    for (int p = 0; p < PPT; ++p) acc[p] += s[p * 256];
+  }
+  const float f = which == 0 ? a.scale : 1.f;
+  const unsigned base = lds_addr(rows);
+#pragma unroll
+  for (int p = 0; p < PPT; ++p) {
+    const int piece = wave + 4 * p;  // 4 db + i
+    bf16x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (bf16)(acc[p][j] * f);
+    lds_write_b64(base + L::byte(lane & 31, piece) + 8 * (lane >> 5), v);
+  }
+  __syncthreads();
+  const int hk = unit % a.Hkv, b = unit / a.Hkv, row0 = kt * 128 + quarter * 32;
+  const int64_t* st = which == 0 ? a.sdk : a.sdv;
+  bf16* dst = (which == 0 ? a.dk : a.dv) + b * st[0] + hk * st[2];
+#pragma unroll
+  for (int k = 0; k < 32 * L::U / 256; ++k) {
+    const int row = (tid + 256 * k) / L::U, u = tid % L::U;
+    if (row0 + row < a.T)
+      __builtin_nontemporal_store(lds_read_b128(base + L::byte(row, u)),
+                                  reinterpret_cast<bf16x8*>(dst + (int64_t)(row0 + row) * st[1] + 8 * u));
+  }
+}
+
+// The chunks of a split dK/dV for these sizes; n = 0 where it does not pay.
+//
+// A key tile's workgroup walks its query tiles one after the other: 1.2 us
+// each at D = 128 and 0.65 us at D = 64 while workgroups have a CU to
+// themselves, so a grid that does not fill the chip takes as long as its
+// longest key tile.  In chunks that fill the workgroup slots once, a query
+// tile takes about 1.5 (D = 128) or 2.5 (D = 64) times that, beside about
+// 8 us for the second prologue, the fp32 partial sums and the merge: the
+// comparison below, in query tiles.  Chunks that fill the slots one and a
+// half or two times, or half, measured slower (B = 2, T = 1777, 12 query on 4
+// kv heads, D = 128, causal: backward 253 us unsplit, 111 us at one filling,
+// 133 / 131 / 126 at 1.5, 2 and 0.5).  Others, backward before and after: B = 1,
+// T = 2048, H = 6, D = 64, causal 71.6 -> 52.6 us; 12 on 4 heads, W = 512
+// 52.5 -> 35.0; 8 on 1, T = 8192 1289 -> 308; T = 8192, 16 on 4, D = 128,
+// W = 2048 504 -> 415; T = 1777, 12 on 12, D = 128 124 -> 112.  Where the rule says no: T = 4096, H = 16, D = 64, causal
+// 154.8 against 159.5 us split.
+DkdvSplit dkdv_split_plan(int B, int T, int H, int Hkv, int D, int W) {
+  constexpr int64_t kMinLen = 16;
+  DkdvSplit s{};
+  const int slots = 256 * (D == 64 ? 3 : 2), G = H / Hkv;
+  const int64_t units = (int64_t)B * Hkv, tiles = ((int64_t)T + 127) / 128;
+  if (units * tiles >= slots) return s;
+  const int nkt = (int)tiles;
+  // Query tiles that key tile kt meets, over the group's heads (never more
+  // than for the key tile before it).
+  auto len = [&](int kt) {
+    const int k0 = kt * 128;
+    return (std::min((int64_t)T - 1, (int64_t)k0 + 126 + W) / 32 - k0 / 32 + 1) * G;
+  };
+  const int64_t longest = len(0);
+  int64_t total = 0;
+  for (int kt = 0; kt < nkt; ++kt) total += len(kt);
+  int64_t c = std::max({(total * units + slots - 1) / slots, (longest + kMaxDkdvChunks - 1) / kMaxDkdvChunks, kMinLen});
+  for (; c < longest; c += std::max(c / 32, (int64_t)1)) {
+    int64_t blocks = 0;
+    for (int kt = 0; kt < nkt; ++kt) blocks += (len(kt) + c - 1) / c;
+    if (blocks * units <= slots) break;
+  }
+  if (D == 64 ? 5 * c + 24 >= 2 * longest : 3 * c + 16 >= 2 * longest) return s;
+  s.len = (int)c;
+  for (; s.n * c < longest; ++s.n) {
+    int has = 0;  // key tiles with a chunk s.n
+    while (has < nkt && len(has) > s.n * c) ++has;
+    s.base[s.n + 1] = s.base[s.n] + has;
+  }
+  return s;
+}
+
 template <int D>
 hipError_t launch_bwd_dkdv(const BwdArgs& a, hipStream_t stream) {
   constexpr int BNK = 4 * 32;
   const int nkt = (a.T + BNK - 1) / BNK;
-  const int64_t blocks = (int64_t)nkt * a.Hkv * a.B;
+  const int64_t units = (int64_t)a.Hkv * a.B;
   // D = 64: six slots of 8 KB (three workgroups per CU), the K/V staging in
   // four of them behind two tiles in flight; D = 128: four slots of 16 KB
   // (two per CU), three tiles in flight from the start.
-  if constexpr (D == 64)
-    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, 6, 2>), dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
-  else
-    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, 4, 3>), dim3((unsigned)blocks), dim3(kThreads), 0, stream, a);
+  constexpr int NBUF = D == 64 ? 6 : 4, PRE = D == 64 ? 2 : 3;
+  if (a.split.n == 0) {
+    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, NBUF, PRE, false>), dim3((unsigned)(nkt * units)), dim3(kThreads), 0, stream, a);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, NBUF, PRE, true>), dim3((unsigned)(a.split.base[a.split.n] * units)),
+                     dim3(kThreads), 0, stream, a);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  const int64_t split_tiles = a.split.base[2] - a.split.base[1];
+  hipLaunchKernelGGL((attn_bwd_dkdv_merge_kernel<D>), dim3((unsigned)(split_tiles * units * 8)), dim3(kThreads), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -65,6 +65,18 @@ struct FwdArgs {
   int nsplit;
 };
 
+// Split dK/dV (attn_bwd_dkdv.hip): the query tiles that a key tile meets are
+// cut into chunks of `len`, one workgroup each.  Chunk c exists for the key
+// tiles 0 .. base[c + 1] - base[c] - 1 (the count of query tiles never grows
+// with the key tile), and its partial sums are block base[c] + key tile of
+// `part`.  n = 0: not split.
+constexpr int kMaxDkdvChunks = 16;
+struct DkdvSplit {
+  float* part;
+  int len, n;
+  int base[kMaxDkdvChunks + 1];
+};
+
 struct BwdArgs {
   const bf16* q;
   const bf16* k;
@@ -80,6 +92,7 @@ struct BwdArgs {
   int B, T, H, Hkv, W;
   float scale;       // softmax scale
   float scale_log2;  // scale * log2(e)
+  DkdvSplit split;
 };
 
 // Arguments of the fused q/k RMSNorm + partial rotary kernels (qk_norm_rope.hip).

@@ -16,6 +16,7 @@ template <int D>
 int fwd_split_count(int B, int T, int H, int W);
 template <int D>
 hipError_t launch_bwd(const BwdArgs& a, hipStream_t stream, int phases);
+DkdvSplit dkdv_split_plan(int B, int T, int H, int Hkv, int D, int W);
 int fused_partial_slots(int T, int W);
 hipError_t launch_bwd_fused(const BwdArgs& a, bf16* part, int R, hipStream_t stream);
 template <int D>
@@ -81,7 +82,7 @@ void copy3(int64_t dst[3], const int64_t* src) {
 
 extern "C" {
 
-int hlm_attn_abi_version(void) { return 8; }
+int hlm_attn_abi_version(void) { return 9; }
 
 const char* hlm_attn_last_error(void) { return g_last_error; }
 
@@ -178,8 +179,16 @@ int check_bwd(const void* q, const void* k, const void* v, const void* o, const 
 }
 
 // phases: kBwdDq / kBwdDkDv / kBwdAll for the two-kernel backward, or
-// kBwdFused (with `part`, `part_bytes`) for the single-pass one.
+// kBwdFused (with `part`, `part_bytes`) for the single-pass one; kBwdAll |
+// kBwdSplit (with `part`, `part_bytes`) cuts long dK/dV tiles into chunks
+// where dkdv_split_plan says so.
 constexpr int kBwdFused = 4;
+constexpr int kBwdSplit = 8;
+
+// Bytes of a split's partial sums: one fp32 dK and dV tile of 128 keys per chunk.
+int64_t split_bytes(const hlm::DkdvSplit& p, int B, int Hkv, int D) {
+  return (int64_t)p.base[p.n] * B * Hkv * 128 * D * 8;
+}
 
 int run_bwd(int phases, const void* q, const void* k, const void* v, const void* o, const void* dout,
             const float* lse, void* dq, void* dk, void* dv, float* delta_ws, int B, int T, int H, int Hkv,
@@ -192,6 +201,17 @@ int run_bwd(int phases, const void* q, const void* k, const void* v, const void*
                      do_strides, dq_strides, dk_strides, dv_strides, scale);
   if (rc) return rc;
   int R = 0;
+  hlm::DkdvSplit split{};
+  if ((phases & kBwdSplit) && B > 0 && T > 0) {
+    split = hlm::dkdv_split_plan(B, T, H, Hkv, D, effective_window(window, T));
+    const int64_t need = split_bytes(split, B, Hkv, D);
+    if (need > 0 && (part == nullptr || !aligned16(part)))
+      return fail(HLM_ATTN_EINVAL, "partial workspace is null or not 16-byte aligned");
+    if (part_bytes < need)
+      return fail(HLM_ATTN_EINVAL, "partial workspace holds %lld bytes, %lld needed", (long long)part_bytes,
+                  (long long)need);
+    split.part = static_cast<float*>(part);
+  }
   if (phases == kBwdFused) {
     if (D != 64) return fail(HLM_ATTN_EUNSUPPORTED, "the single-pass backward takes head_dim 64 only (got %d)", D);
     if (B == 0 || T == 0) return HLM_ATTN_OK;
@@ -230,6 +250,7 @@ int run_bwd(int phases, const void* q, const void* k, const void* v, const void*
   a.W = effective_window(window, T);
   a.scale = scale;
   a.scale_log2 = scale * hlm::kLog2e;
+  a.split = split;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const hipError_t err = phases == kBwdFused ? hlm::launch_bwd_fused(a, static_cast<hlm::bf16*>(part), R, s)
                          : D == 64           ? hlm::launch_bwd<64>(a, s, phases)
@@ -338,6 +359,22 @@ extern "C" {
 int hlm_attn_bwd(HLM_BWD_PARAMS) { return run_bwd(hlm::kBwdAll, HLM_BWD_ARGS); }
 int hlm_attn_bwd_dq(HLM_BWD_PARAMS) { return run_bwd(hlm::kBwdDq, HLM_BWD_ARGS); }
 int hlm_attn_bwd_dkdv(HLM_BWD_PARAMS) { return run_bwd(hlm::kBwdDkDv, HLM_BWD_ARGS); }
+
+int64_t hlm_attn_bwd_split_workspace_bytes(int B, int T, int H, int Hkv, int D, int window) {
+  g_last_error[0] = '\0';
+  if (const int rc = check_dims(B, T, H, Hkv, D, 1.f)) return rc;
+  if (B == 0 || T == 0) return 0;
+  return split_bytes(hlm::dkdv_split_plan(B, T, H, Hkv, D, effective_window(window, T)), B, Hkv, D);
+}
+
+int hlm_attn_bwd_split(const void* q, const void* k, const void* v, const void* o, const void* dout,
+                       const float* lse, void* dq, void* dk, void* dv, float* delta_ws, void* partial_ws,
+                       int64_t partial_ws_bytes, int B, int T, int H, int Hkv, int D, const int64_t* q_strides,
+                       const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
+                       const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
+                       const int64_t* dv_strides, int window, float scale, void* stream) {
+  return run_bwd(hlm::kBwdAll | kBwdSplit, HLM_BWD_ARGS, partial_ws, partial_ws_bytes);
+}
 
 int64_t hlm_attn_bwd_fused_workspace_bytes(int B, int T, int H, int D, int window) {
   g_last_error[0] = '\0';

@@ -10,7 +10,8 @@ torch's caching allocator, launch on torch's current stream and never
 synchronise.  There is no CPU implementation: on a tensor that is not on a
 ROCm device, or without libhlm_attn.so, the ops raise.
 
-The backward runs the two-kernel path (hlm_attn_bwd: dq, then dkdv) unless
+The backward runs the two-kernel path (hlm_attn_bwd_split: dq, then dkdv, in
+chunks with a merge where the grid is small and its rows are long) unless
 HLM_ATTN_BWD=fused selects the single-pass one (hlm_attn_bwd_fused, head
 dim 64 only; other head dims keep the two-kernel path).
 """
@@ -226,13 +227,34 @@ def hip_attn_bwd(
                 B, T, H, Hkv, D, *strides, int(window), float(scale), _stream_handle(q.device),
             )
         else:
-            rc = lib.hlm_attn_bwd(
+            nbytes = bwd_split_bytes(B, T, H, Hkv, D, int(window))
+            part = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+            rc = lib.hlm_attn_bwd_split(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(), lse.data_ptr(),
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr(),
+                None if part is None else part.data_ptr(), nbytes,
                 B, T, H, Hkv, D, *strides, int(window), float(scale), _stream_handle(q.device),
             )
     _lib.check(rc, lib)
     return dq, dk, dv
+
+
+_bwd_split_cache: dict = {}
+
+
+def bwd_split_bytes(B: int, T: int, H: int, Hkv: int, D: int, window: int) -> int:
+    """hlm_attn_bwd_split_workspace_bytes, memoised per shape."""
+    key = (B, T, H, Hkv, D, window)
+    n = _bwd_split_cache.get(key)
+    if n is None:
+        lib = _lib.load()
+        n = lib.hlm_attn_bwd_split_workspace_bytes(*key)
+        if n < 0:
+            _lib.check(n, lib)
+        if len(_bwd_split_cache) > 4096:
+            _bwd_split_cache.clear()
+        _bwd_split_cache[key] = n
+    return n
 
 
 def fused_backward_selected() -> bool:

@@ -1,0 +1,123 @@
+"""The backward with long dK/dV tiles cut into chunks (hlm_attn_bwd_split): its
+argument checks and the shapes it applies to (CPU), and its results against
+hlm_attn_bwd and the fp32 oracle (GPU).
+
+dq comes from the same kernel and must be bit-identical.  dk and dv are the
+same fp32 products summed in another order and rounded to bf16 once, so two
+results differ by at most one bf16 step of the value (2^-7 relative) plus the
+fp32 sums' own reordering error, which is far below 1e-5 of the largest
+gradient.  Every call starts from a NaN-filled workspace.
+"""
+from __future__ import annotations
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+from hlm_attn import _lib
+from oracle import attention as oracle
+from test_gpu_parity import assert_grad, make_inputs
+
+CASES = [
+    # B, T, H, Hkv, D, window
+    (1, 1, 64, 1, 64, None),      # one token, one key tile, 64 query heads: chunks of whole heads
+    (1, 129, 32, 1, 128, None),   # a second key tile of one row
+    (1, 300, 40, 2, 64, 40),      # short window, many heads: chunks end inside a head
+    (1, 777, 16, 1, 128, None),   # ragged, causal: key tiles with 1 to 16 chunks
+    (2, 1025, 12, 4, 64, None),
+    (1, 1500, 8, 2, 128, 700),    # windowed: the rotated tile order across chunks
+    (2, 1777, 12, 4, 128, None),
+    (1, 2048, 6, 6, 64, None),    # no grouping
+]
+
+
+def _bytes(B, T, H, Hkv, D, window):
+    return _lib.load().hlm_attn_bwd_split_workspace_bytes(B, T, H, Hkv, D, window or 0)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_split_applies_to_the_cases_below(case):
+    B, T, H, Hkv, D, _ = case
+    tiles, n = (T + 127) // 128, _bytes(*case)
+    block = B * Hkv * 128 * D * 8  # one chunk of every (batch, kv head): fp32 dK and dV of 128 keys
+    assert n % block == 0 and 2 * block <= n <= 16 * tiles * block
+    assert n // (128 * D * 8) <= 256 * (3 if D == 64 else 2), "at most one filling of the chip"
+
+
+@pytest.mark.parametrize(
+    "case",
+    [
+        (8, 2048, 12, 12, 64, 512),    # the chip is full
+        (1, 16384, 16, 16, 128, 2048),
+        (1, 1000, 6, 6, 64, 300),      # short rows
+        (1, 333, 4, 1, 64, 129),
+        (1, 4096, 16, 16, 64, None),   # chunks would be as long as the slots they fill are slow
+        (0, 128, 2, 2, 64, None),
+    ],
+)
+def test_split_does_not_apply(case):
+    assert _bytes(*case) == 0
+
+
+def test_split_backward_checks_its_workspace():
+    lib = _lib.load()
+    assert lib.hlm_attn_bwd_split_workspace_bytes(1, 128, 3, 2, 64, 0) == -1
+    assert lib.hlm_attn_bwd_split_workspace_bytes(1, 128, 2, 2, 96, 0) == -2
+    T, H, D = 129, 32, 128
+    need = _bytes(1, T, H, 1, D, None)
+    s, p = (ctypes.c_int64 * 3)(T * H * D, H * D, D), ctypes.c_void_p(0x1000)
+
+    def call(ws, n):
+        return lib.hlm_attn_bwd_split(*([p] * 10), ws, n, 1, T, H, 1, D, *([s] * 8), 0, 0.1, None)
+
+    assert call(None, need) == -1 and b"partial workspace" in lib.hlm_attn_last_error()
+    assert call(ctypes.c_void_p(0x1008), need) == -1
+    assert call(p, need - 1) == -1 and b"needed" in lib.hlm_attn_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES)
+def test_split_backward_matches_the_unsplit_one_and_the_oracle(case):
+    from hlm_attn import ops
+
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm device")
+    dev = torch.device("cuda", 0)
+    B, T, H, Hkv, D, window = case
+    print(f"case split B={B} T={T} H={H} Hkv={Hkv} D={D} W={window}", flush=True)
+    q, k, v, do = make_inputs(B, T, H, Hkv, D, 70 + T)
+    qd, kd, dod = (t.to(dev) for t in (q, k, do))
+    vd = torch.empty(B, T, 2 * Hkv, D, dtype=torch.bfloat16, device=dev)[:, :, Hkv:]  # a strided view
+    vd.copy_(v)
+    w, scale, lib = window or 0, 1.0 / math.sqrt(D), _lib.load()
+    o, lse = ops.hip_attn_fwd(qd, kd, vd, w, scale)
+    n = _bytes(*case)
+    got = []
+    for split in (False, True, True):
+        dq, dk, dv = (torch.full_like(t, float("nan"), memory_format=torch.contiguous_format) for t in (qd, kd, vd))
+        delta = torch.empty(2 * B * H * T, device=dev)
+        part = torch.full((n // 4,), float("nan"), device=dev)
+        ptrs = [t.data_ptr() for t in (qd, kd, vd, o, dod, lse, dq, dk, dv, delta)]
+        st = [_lib.strides3(t) for t in (qd, kd, vd, o, dod, dq, dk, dv)]
+        tail = (B, T, H, Hkv, D, *st, w, scale, ops._stream_handle(dev))
+        if split:
+            rc = lib.hlm_attn_bwd_split(*ptrs, part.data_ptr(), n, *tail)
+        else:
+            rc = lib.hlm_attn_bwd(*ptrs, *tail)
+        _lib.check(rc, lib)
+        torch.cuda.synchronize()
+        got.append((dq, dk, dv))
+    one, two, again = got
+    assert torch.equal(one[0], two[0])
+    assert all(torch.equal(a, b) for a, b in zip(two, again)), "not deterministic"
+    for name, a, b in (("dk", one[1], two[1]), ("dv", one[2], two[2])):
+        a, b = a.float(), b.float()
+        assert bool(((a - b).abs() <= 2.0**-7 * a.abs() + 1e-5 * a.abs().max()).all()), name
+    via_op = ops.hip_attn_bwd(dod, qd, kd, vd, o, lse, w, scale)
+    assert all(torch.equal(a, b) for a, b in zip(two, via_op)), "the op takes the split path"
+    if H * T <= 16 * 1024:
+        rdq, rdk, rdv = oracle.backward(q, k, v, do, window)
+        for name, a, r in zip(("dq", "dk", "dv"), two, (rdq, rdk, rdv)):
+            assert_grad(name, a.float().cpu(), r)
