@@ -12,13 +12,17 @@
 // other target outside [0, V) yields NaN for the row's loss and gradient (the
 // kernel cannot raise).
 //
-// Memory-bound: one workgroup per row.  When rows are 16-byte aligned (V and
-// the row stride multiples of 16 / sizeof(T)), the row is read once into
-// registers in 16-byte chunks (chunk k of thread i holds elements
-// 16/sizeof(T) * (i + 256 k) ..), reduced (max, then sum of exponentials) with
-// wave shuffles and one LDS exchange between the 4 waves, and written once:
-// 2 * V * sizeof(T) bytes per row.  Other layouts take a generic path that
-// reads the row three times (max, sum, write), one element per lane.
+// Memory-bound: one workgroup per row.  The row is read once into registers in
+// the aligned 16-byte chunks that hold it (chunk k of thread i is the row's
+// chunk i + 256 k), reduced (max, then sum of exponentials) with wave shuffles
+// and one LDS exchange between the 4 waves, and written once: 2 * V * sizeof(T)
+// bytes per row.  A row may begin and end inside a chunk (V or the row stride
+// no multiple of 16 / sizeof(T)): the elements of a chunk that are not the
+// row's read as -inf, which neither the maximum nor the sum sees, and are not
+// written.  4096 rows of V = 50257 bf16 at a row stride of 50257: 529 us when
+// such rows were read three times, one element per lane; 169 us now (4.9 TB/s).  Rows
+// of more than 32 chunks per thread (V above 65528 bf16 or 32764 fp32) keep
+// that path.
 #include "attn_common.h"
 
 namespace hlm {
@@ -67,9 +71,17 @@ __device__ __forceinline__ int target_status(int64_t t, int V, int ignore_index)
   return t == ignore_index ? 1 : 2;
 }
 
-template <typename T, int K>
+// ALIGNED: every row begins and ends on a 16-byte boundary.
+template <typename T, int K, bool ALIGNED>
 __global__ __launch_bounds__(256) void ce_rows_vec_kernel(CeArgs a) {
   constexpr int E = 16 / sizeof(T);  // elements per 16-byte chunk
+  // LEAN: one buffer resource and offset register for all chunks, and nothing
+  // derived from a chunk is kept over the reductions (they cost 11 VGPRs a
+  // chunk otherwise: one wave per SIMD from K = 24 on).  4096 rows of bf16, us
+  // without / with: V = 65536 273 / 213, V = 50264 216 / 167, V = 50257
+  // (unaligned) 231 / 169, V = 16381 64.5 / 52.5.  Aligned rows of up to 16
+  // chunks run best without, at two waves per SIMD: V = 32768 95 / 108.
+  constexpr bool LEAN = !ALIGNED || K > 16;
   typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
   __shared__ float red[4];
   const int row = blockIdx.x, tid = threadIdx.x;
@@ -77,6 +89,13 @@ __global__ __launch_bounds__(256) void ce_rows_vec_kernel(CeArgs a) {
   const int V = a.V;
   const int64_t tgt = a.targets[row];
   const int status = target_status(tgt, V, a.ignore_index);
+  // The row's elements are E * chunk - lead + e, 0 <= lead < E.
+  const int lead = ALIGNED ? 0 : (int)((reinterpret_cast<uintptr_t>(base) & 15u) / sizeof(T));
+  auto first_of = [&](int k) __attribute__((always_inline)) { return E * (tid + 256 * k) - lead; };
+  // Buffer over the row from its first chunk to its last 4 bytes (reads past
+  // them return zeros).
+  [[maybe_unused]] const __amdgpu_buffer_rsrc_t chunks =
+      bytes_rsrc(base - lead, ((V + lead) * (int)sizeof(T) + 3) & ~3);
   // The target's logit, read before any thread of the block stores (the
   // stores follow two block barriers).
   float xt = 0.f;
@@ -86,26 +105,53 @@ __global__ __launch_bounds__(256) void ce_rows_vec_kernel(CeArgs a) {
   float m = -INFINITY;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int idx = E * (tid + 256 * k);
+    const int idx = first_of(k);
     raw[k] = u32x4{};
-    if (idx < V) raw[k] = *reinterpret_cast<const u32x4*>(base + idx);
+    if (idx >= V) continue;
+    if constexpr (LEAN)
+      raw[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(chunks, 16 * tid, 4096 * k, 0));
+    else
+      raw[k] = *reinterpret_cast<const u32x4*>(base + idx);
+  }
+  if constexpr (!ALIGNED) {
+    // The first chunk and the one that holds the row's end: what is not the
+    // row's (a neighbouring row's elements, possibly being written) goes out.
+    auto trim = [&](u32x4& w, int idx) __attribute__((always_inline)) {
+      T* v = reinterpret_cast<T*>(&w);
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if ((unsigned)(idx + e) >= (unsigned)V) v[e] = (T)-INFINITY;
+    };
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int idx = first_of(k);
+      if (idx < 0 || (idx < V && idx + E > V)) trim(raw[k], idx);
+    }
   }
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    if (E * (tid + 256 * k) >= V) continue;
+    if (first_of(k) >= V) continue;
     const T* v = reinterpret_cast<const T*>(&raw[k]);
 #pragma unroll
     for (int e = 0; e < E; ++e) m = fmaxf(m, to_f32(v[e]));
+  }
+  if constexpr (LEAN) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) asm volatile("" : "+v"(raw[k]));
   }
   const float M = block_max(m, red);
   const float c = M * kLog2e;
   float s = 0.f;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    if (E * (tid + 256 * k) >= V) continue;
+    if (first_of(k) >= V) continue;
     const T* v = reinterpret_cast<const T*>(&raw[k]);
 #pragma unroll
     for (int e = 0; e < E; ++e) s += fast_exp2(fmaf(to_f32(v[e]), kLog2e, -c));
+  }
+  if constexpr (LEAN) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) asm volatile("" : "+v"(raw[k]));
   }
   const float S = block_sum(s, red);
   const float lse = M + __log2f(S) * kLn2;
@@ -114,7 +160,7 @@ __global__ __launch_bounds__(256) void ce_rows_vec_kernel(CeArgs a) {
   const float scale = status == 0 ? a.inv_n / S : status == 1 ? 0.f : NAN;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int idx = E * (tid + 256 * k);
+    const int idx = first_of(k);
     if (idx >= V) continue;
     const T* v = reinterpret_cast<const T*>(&raw[k]);
     u32x4 outw;
@@ -130,7 +176,16 @@ __global__ __launch_bounds__(256) void ce_rows_vec_kernel(CeArgs a) {
       for (int e = 0; e < E; ++e)
         if (e == et) o[e] = (T)(fast_exp2(fmaf(to_f32(v[e]), kLog2e, -c)) * scale - a.inv_n);
     }
-    *reinterpret_cast<u32x4*>(base + idx) = outw;
+    if (ALIGNED || (idx >= 0 && idx + E <= V)) {
+      if constexpr (LEAN)
+        __builtin_amdgcn_raw_buffer_store_b128(outw, chunks, 16 * tid, 4096 * k, 0);
+      else
+        *reinterpret_cast<u32x4*>(base + idx) = outw;
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if ((unsigned)(idx + e) < (unsigned)V) base[idx + e] = o[e];
+    }
   }
 }
 
@@ -161,41 +216,49 @@ __global__ __launch_bounds__(256) void ce_rows_generic_kernel(CeArgs a) {
   }
 }
 
-template <typename T>
-hipError_t launch_ce_rows_typed(const CeArgs& a, bool vec, hipStream_t stream) {
+template <typename T, int K>
+void launch_ce_rows_vec(const CeArgs& a, bool aligned, hipStream_t stream) {
   const dim3 grid((unsigned)a.n_rows), block(256);
-  if (!vec) {
-    hipLaunchKernelGGL((ce_rows_generic_kernel<T>), grid, block, 0, stream, a);
-    return hipGetLastError();
-  }
-  constexpr int E = 16 / sizeof(T);
-  const int chunks = (a.V + 256 * E - 1) / (256 * E);  // 16-byte chunks per thread
-  if (chunks <= 1)
-    hipLaunchKernelGGL((ce_rows_vec_kernel<T, 1>), grid, block, 0, stream, a);
-  else if (chunks <= 2)
-    hipLaunchKernelGGL((ce_rows_vec_kernel<T, 2>), grid, block, 0, stream, a);
-  else if (chunks <= 4)
-    hipLaunchKernelGGL((ce_rows_vec_kernel<T, 4>), grid, block, 0, stream, a);
-  else if (chunks <= 8)
-    hipLaunchKernelGGL((ce_rows_vec_kernel<T, 8>), grid, block, 0, stream, a);
-  else if (chunks <= 16)
-    hipLaunchKernelGGL((ce_rows_vec_kernel<T, 16>), grid, block, 0, stream, a);
-  else if (chunks <= 32)
-    hipLaunchKernelGGL((ce_rows_vec_kernel<T, 32>), grid, block, 0, stream, a);
+  if (aligned)
+    hipLaunchKernelGGL((ce_rows_vec_kernel<T, K, true>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((ce_rows_generic_kernel<T>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((ce_rows_vec_kernel<T, K, false>), grid, block, 0, stream, a);
+}
+
+template <typename T>
+hipError_t launch_ce_rows_typed(const CeArgs& a, hipStream_t stream) {
+  constexpr int E = 16 / sizeof(T);
+  const bool aligned = (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0 && a.V % E == 0 && a.row_stride % E == 0;
+  // 16-byte chunks per thread; a row that is not aligned may reach into one more.
+  const int chunks = (int)(((int64_t)a.V + (aligned ? 0 : E - 1) + 256 * E - 1) / (256 * E));
+  if (chunks <= 1)
+    launch_ce_rows_vec<T, 1>(a, aligned, stream);
+  else if (chunks <= 2)
+    launch_ce_rows_vec<T, 2>(a, aligned, stream);
+  else if (chunks <= 4)
+    launch_ce_rows_vec<T, 4>(a, aligned, stream);
+  else if (chunks <= 8)
+    launch_ce_rows_vec<T, 8>(a, aligned, stream);
+  else if (chunks <= 16)
+    launch_ce_rows_vec<T, 16>(a, aligned, stream);
+  else if (chunks <= 20)
+    launch_ce_rows_vec<T, 20>(a, aligned, stream);
+  else if (chunks <= 24)
+    launch_ce_rows_vec<T, 24>(a, aligned, stream);
+  else if (chunks <= 28)
+    launch_ce_rows_vec<T, 28>(a, aligned, stream);
+  else if (chunks <= 32)
+    launch_ce_rows_vec<T, 32>(a, aligned, stream);
+  else
+    hipLaunchKernelGGL((ce_rows_generic_kernel<T>), dim3((unsigned)a.n_rows), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
-// Entry from the C ABI: rows are 16-byte aligned when the base, V and the row
-// stride allow it (then the register-resident path is used).
 hipError_t launch_ce_rows(void* logits, bool bf16_logits, int64_t row_stride, const int64_t* targets, float* loss,
                           int n_rows, int V, float inv_n, int ignore_index, hipStream_t stream) {
   CeArgs a{logits, row_stride, targets, loss, n_rows, V, inv_n, ignore_index};
   if (n_rows == 0) return hipSuccess;
-  const int E = bf16_logits ? 8 : 4;
-  const bool vec = (reinterpret_cast<uintptr_t>(logits) & 15u) == 0 && V % E == 0 && row_stride % E == 0;
-  return bf16_logits ? launch_ce_rows_typed<bf16>(a, vec, stream) : launch_ce_rows_typed<float>(a, vec, stream);
+  return bf16_logits ? launch_ce_rows_typed<bf16>(a, stream) : launch_ce_rows_typed<float>(a, stream);
 }
 
 }  // namespace hlm
