@@ -23,6 +23,10 @@ template <int D>
 hipError_t launch_qk_norm_rope(const QkNormRopeArgs& a, bool backward, hipStream_t stream);
 hipError_t launch_ce_rows(void* logits, bool bf16_logits, int64_t row_stride, const int64_t* targets, float* loss,
                           int n_rows, int V, float inv_n, int ignore_index, hipStream_t stream);
+int lm_head_dhidden_runs(int M, int N, int K);
+bool lm_head_dhidden_pays(int M, int N, int K);
+hipError_t launch_lm_head_dhidden(const void* g, int64_t ldg, const void* w, int64_t ldw, void* c, int64_t ldc, float* part,
+                                  int M, int N, int K, hipStream_t stream);
 hipError_t launch_residual_rms_norm(const void* a, const void* b, const void* c, void* y0, void* y1, int64_t rows,
                                     int n, float eps, bool backward, hipStream_t stream);
 }  // namespace hlm
@@ -82,7 +86,7 @@ void copy3(int64_t dst[3], const int64_t* src) {
 
 extern "C" {
 
-int hlm_attn_abi_version(void) { return 9; }
+int hlm_attn_abi_version(void) { return 10; }
 
 const char* hlm_attn_last_error(void) { return g_last_error; }
 
@@ -487,6 +491,70 @@ int hlm_ce_rows(void* logits, int logits_dtype, int64_t row_stride, const int64_
                                              n_cols, (float)(1.0 / (double)n_tokens), ignore_index,
                                              static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(HLM_ATTN_ELAUNCH, "cross-entropy launch failed: %s", hipGetErrorString(err));
+  return HLM_ATTN_OK;
+}
+
+}  // extern "C"
+
+namespace {
+
+int check_ce_dhidden(int n_rows, int n_hidden, int n_vocab) {
+  if (n_rows < 0 || n_hidden <= 0 || n_vocab <= 0)
+    return fail(HLM_ATTN_EINVAL, "bad shape n_rows=%d n_hidden=%d n_vocab=%d", n_rows, n_hidden, n_vocab);
+  if (n_hidden % 8 != 0) return fail(HLM_ATTN_EUNSUPPORTED, "n_hidden %d is not a multiple of 8", n_hidden);
+  // workgroups (rows / 256 x hidden / 256 tiles) and their 32-bit byte offsets
+  if (n_hidden > (1 << 20) || n_vocab > (1 << 21))
+    return fail(HLM_ATTN_EUNSUPPORTED, "n_hidden %d or n_vocab %d is too large", n_hidden, n_vocab);
+  if ((((int64_t)n_rows + 255) / 256) * (((int64_t)n_hidden + 255) / 256) >= (1 << 20))
+    return fail(HLM_ATTN_EUNSUPPORTED, "problem too large for one launch");
+  return HLM_ATTN_OK;
+}
+
+int64_t ce_dhidden_bytes(int n_rows, int n_hidden, int n_vocab) {
+  const int runs = hlm::lm_head_dhidden_runs(n_rows, n_hidden, n_vocab);
+  return runs == 1 ? 0 : (int64_t)runs * ((n_rows + 255) / 256) * ((n_hidden + 255) / 256) * (256 * 256 * 4);
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t hlm_ce_dhidden_workspace_bytes(int n_rows, int n_hidden, int n_vocab) {
+  g_last_error[0] = '\0';
+  if (const int rc = check_ce_dhidden(n_rows, n_hidden, n_vocab)) return rc;
+  return n_rows == 0 ? 0 : ce_dhidden_bytes(n_rows, n_hidden, n_vocab);
+}
+
+int hlm_ce_dhidden_pays(int n_rows, int n_hidden, int n_vocab) {
+  g_last_error[0] = '\0';
+  if (n_rows <= 0 || check_ce_dhidden(n_rows, n_hidden, n_vocab) != HLM_ATTN_OK) return 0;
+  return hlm::lm_head_dhidden_pays(n_rows, n_hidden, n_vocab) ? 1 : 0;
+}
+
+int hlm_ce_dhidden(const void* grad, int64_t grad_stride, const void* weight, int64_t weight_stride, void* dhidden,
+                   int64_t dhidden_stride, int n_rows, int n_hidden, int n_vocab, void* ws, int64_t ws_bytes,
+                   void* stream) {
+  g_last_error[0] = '\0';
+  if (const int rc = check_ce_dhidden(n_rows, n_hidden, n_vocab)) return rc;
+  const int64_t padded = ((int64_t)n_vocab + 63) / 64 * 64;
+  if (grad_stride < padded || grad_stride % 8 != 0 || grad_stride > (1 << 21))
+    return fail(HLM_ATTN_EINVAL, "grad stride %lld must be a multiple of 8 in [%lld, 2^21]", (long long)grad_stride,
+                (long long)padded);
+  if (weight_stride < n_hidden || weight_stride % 8 != 0 || weight_stride > (1 << 22))
+    return fail(HLM_ATTN_EINVAL, "weight stride %lld must be a multiple of 8 in [%d, 2^22]", (long long)weight_stride, n_hidden);
+  if (dhidden_stride < n_hidden || dhidden_stride % 8 != 0)
+    return fail(HLM_ATTN_EINVAL, "dhidden stride %lld must be a multiple of 8 and at least %d", (long long)dhidden_stride,
+                n_hidden);
+  if (n_rows == 0) return HLM_ATTN_OK;
+  const int64_t need = ce_dhidden_bytes(n_rows, n_hidden, n_vocab);
+  for (const void* p : {grad, weight, static_cast<const void*>(dhidden), need > 0 ? static_cast<const void*>(ws) : grad})
+    if (p == nullptr || !aligned16(p)) return fail(HLM_ATTN_EINVAL, "a pointer is null or not 16-byte aligned");
+  if (ws_bytes < need)
+    return fail(HLM_ATTN_EINVAL, "workspace holds %lld bytes, %lld needed", (long long)ws_bytes, (long long)need);
+  const hipError_t err =
+      hlm::launch_lm_head_dhidden(grad, grad_stride, weight, weight_stride, dhidden, dhidden_stride, static_cast<float*>(ws),
+                                  n_rows, n_hidden, n_vocab, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(HLM_ATTN_ELAUNCH, "dhidden launch failed: %s", hipGetErrorString(err));
   return HLM_ATTN_OK;
 }
 

@@ -462,6 +462,41 @@ def _(logits, targets, n_tokens):
     return logits.new_empty((logits.shape[0],), dtype=torch.float32)
 
 
+def _ce_dhidden_ready(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> bool:
+    """True where hlm_ce_dhidden takes these tensors and beats the library's product."""
+    if not all(t.is_cuda and t.dtype is _BF16 and t.stride(1) == 1 and not (t.stride(0) & 7 or t.data_ptr() & 15)
+               for t in (work, weight, out)):
+        return False
+    return _lib.load().hlm_ce_dhidden_pays(work.shape[0], weight.shape[1], n_vocab) == 1
+
+
+@torch.library.custom_op("hackable_lm::hip_ce_dhidden", mutates_args=("out",))
+def hip_ce_dhidden(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> None:
+    """out = work[:, :n_vocab] @ weight, where work's columns from n_vocab to the
+    next multiple of 64 hold zeros.  The choice between hlm_ce_dhidden and the
+    library's product is made here, so that a trace holds one op."""
+    rows, n = work.shape[0], weight.shape[1]
+    if weight.shape[0] != n_vocab or out.shape != (rows, n) or work.shape[1] < -(-n_vocab // 64) * 64:
+        raise RuntimeError(f"work {tuple(work.shape)}, weight {tuple(weight.shape)} and out {tuple(out.shape)} do not match")
+    if not _ce_dhidden_ready(work, weight, n_vocab, out):
+        torch.mm(work[:, :n_vocab], weight, out=out)
+        return
+    lib = _lib.load()
+    nbytes = lib.hlm_ce_dhidden_workspace_bytes(rows, n, n_vocab)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=work.device) if nbytes else None
+    with _on_device(work.device):
+        rc = lib.hlm_ce_dhidden(
+            work.data_ptr(), work.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(), out.stride(0),
+            rows, n, n_vocab, None if ws is None else ws.data_ptr(), nbytes, _stream_handle(work.device),
+        )
+    _lib.check(rc, lib)
+
+
+@hip_ce_dhidden.register_fake
+def _(work, weight, n_vocab, out):
+    return None
+
+
 # --- residual add + RMSNorm after the output / down projections -------------------
 #
 # hackable_lm::hip_residual_rms_norm computes residual_rms_norm

@@ -263,14 +263,34 @@ int hlm_qk_norm_rope_bwd(const void* q, const void* k, const void* grad_q_out, c
  *                                                           the mean loss)
  * computed in fp32.  A target equal to ignore_index gives a zero loss and a
  * zero gradient row (F.cross_entropy's rule); any other target outside
- * [0, n_cols) gives NaN for that row.  16-byte aligned rows (logits, n_cols
- * and row_stride multiples of 16 bytes) take a path that reads and writes
- * each row once.  Replaces the hackable_lm::linear_ce Triton op and its
+ * [0, n_cols) gives NaN for that row.  Rows of up to 65528 bf16 or 32764 fp32
+ * values, whatever their alignment, are read and written once.  Replaces the hackable_lm::linear_ce Triton op and its
  * kernel (/root/reference/kernels.py:286-336) inside the chunked fused
  * linear cross-entropy (/root/reference/kernels.py:878-959).
  */
 int hlm_ce_rows(void* logits, int logits_dtype, int64_t row_stride, const int64_t* targets, float* loss, int n_rows,
                 int n_cols, int64_t n_tokens, int ignore_index, void* stream);
+
+/*
+ * dhidden of the same chunk: dhidden = grad weight with fp32 sums, all bf16:
+ * grad (n_rows x n_vocab, hlm_ce_rows' gradients), weight (n_vocab x
+ * n_hidden) and dhidden (n_rows x n_hidden), rows at the given strides in
+ * elements.  The columns n_vocab .. round_up(n_vocab, 64) - 1 of grad's rows
+ * must exist and hold zeros.  n_hidden and the strides are multiples of 8, the
+ * pointers 16-byte aligned.  Several workgroups share an output tile and their
+ * fp32 partial tiles, added in a fixed order, lie in ws: hlm_ce_dhidden_
+ * workspace_bytes (0 possible), 16-byte aligned, no initialisation needed.
+ * Stands where the reference calls its library product
+ * (/root/reference/kernels.py:878-942).
+ */
+int hlm_ce_dhidden(const void* grad, int64_t grad_stride, const void* weight, int64_t weight_stride, void* dhidden,
+                   int64_t dhidden_stride, int n_rows, int n_hidden, int n_vocab, void* ws, int64_t ws_bytes,
+                   void* stream);
+/* Bytes of hlm_ce_dhidden's workspace; negative: an HLM_ATTN_E* code. */
+int64_t hlm_ce_dhidden_workspace_bytes(int n_rows, int n_hidden, int n_vocab);
+/* 1 where hlm_ce_dhidden takes the sizes and beats a product that does not
+ * split the sum over the vocabulary, else 0.  Pure function of the sizes. */
+int hlm_ce_dhidden_pays(int n_rows, int n_hidden, int n_vocab);
 
 /*
  * Residual add + RMSNorm (no weight) after an output or down projection:
