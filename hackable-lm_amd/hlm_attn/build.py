@@ -116,11 +116,12 @@ def build_torch_fwd() -> Path:
     if cxx is None:
         raise RuntimeError("no host C++ compiler (g++) for the torch extension")
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
-    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-w",
+    rocm = Path(hipcc()).resolve().parent.parent
+    cmd = [cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DTORCH_EXTENSION_NAME=_torch_fwd", "-DTORCH_API_INCLUDE_EXTENSION_H",
-           *[f"-I{d}" for d in cpp_extension.include_paths()], f"-I{sysconfig.get_paths()['include']}",
+           *[f"-I{d}" for d in cpp_extension.include_paths()], f"-I{rocm / 'include'}", f"-I{sysconfig.get_paths()['include']}",
            str(CSRC / "torch_fwd.cpp"),
-           *[f"-L{d}" for d in cpp_extension.library_paths()], "-lc10", "-ltorch", "-ltorch_cpu", "-ltorch_python",
+           *[f"-L{d}" for d in cpp_extension.library_paths()], "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python",
            f"-L{PKG_DIR}", "-lhlm_attn", "-Wl,-rpath,$ORIGIN"]
     tmp = TORCH_FWD_PATH.with_name(TORCH_FWD_PATH.name + ".tmp")
     _run([*cmd, "-o", str(tmp)])

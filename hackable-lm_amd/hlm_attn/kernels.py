@@ -107,7 +107,10 @@ def attention(
     if ops.direct_call_ok(q, k, v):  # inference: same kernels, without the dispatcher's host cost
         out, _ = ops.attn_fwd_impl(q, k, v, window, float(scale))
     else:
-        out, _ = ops.hip_attn_fwd(q, k, v, window, float(scale))
+        ext = ops.eager_ext(q, k, v)
+        out = ext.attn_train(q, k, v, window, float(scale)) if ext is not None else None
+        if out is None:
+            out, _ = ops.hip_attn_fwd(q, k, v, window, float(scale))
     return out if d_kernel == dv else out[..., :dv]
 
 
@@ -211,6 +214,10 @@ def qk_norm_rope_hip(
         raise RuntimeError("qk_norm_rope_hip runs on ROCm devices only; use the torch path on the CPU")
     if ops.direct_call_ok(q, k, cos, sin):  # inference: same kernel, without the dispatcher's host cost
         return ops.qk_norm_rope_impl(q, k, cos, sin, float(eps))
+    ext = ops.eager_ext(q, k, cos, sin)
+    out = ext.qk_norm_rope_train(q, k, cos, sin, float(eps)) if ext is not None else None
+    if out is not None:
+        return out
     return ops.hip_qk_norm_rope(q, k, cos, sin, float(eps))
 
 
@@ -344,4 +351,8 @@ def residual_rms_norm_hip(residual: torch.Tensor, branch: torch.Tensor, eps: flo
         raise RuntimeError("residual_rms_norm_hip runs on ROCm devices only; use the torch path on the CPU")
     if ops.direct_call_ok(residual, branch):  # inference: same kernel, without the dispatcher's host cost
         return ops.residual_rms_norm_impl(residual, branch, float(eps))
+    ext = ops.eager_ext(residual, branch)
+    out = ext.residual_rms_norm_train(residual, branch, float(eps)) if ext is not None else None
+    if out is not None:
+        return out
     return ops.hip_residual_rms_norm(residual, branch, float(eps))

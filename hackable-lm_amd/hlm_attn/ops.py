@@ -22,6 +22,7 @@ import ctypes
 import os
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -109,6 +110,24 @@ def direct_call_ok(*tensors: torch.Tensor) -> bool:
         if type(t) is not torch.Tensor or (grad and t.requires_grad):
             return False
     return True
+
+
+def eager_ext(*tensors: torch.Tensor):
+    """The torch extension where a differentiable call may run as one of its
+    C++ autograd functions instead of the custom op, else None: plain tensors
+    and parameters, and nothing active that has to see the op itself (tracing,
+    a dispatch or function mode, a function transform, forward-mode AD)."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
+            or forward_ad._current_level >= 0):
+        return None
+    for t in tensors:
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return None
+    ext = _lib._torch_fwd
+    if ext is None:
+        ext = _lib.torch_fwd()
+    return ext or None
 
 
 def attn_fwd_impl(
