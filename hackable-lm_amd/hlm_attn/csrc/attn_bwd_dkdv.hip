@@ -3,9 +3,9 @@
 // and conventions are described there).
 //
 // This file is compiled with LLVM's default (max-occupancy) machine
-// scheduler, which honours the sched_group_barrier pipeline of the S/dP
-// operand reads below within three waves per SIMD at D = 64; the dQ kernel
-// keeps the iterative-ILP scheduler, which measured 2-5% faster for it.
+// scheduler, which honours the sched_group_barrier pipelines of the operand
+// reads below within three waves per SIMD at D = 64 and two at D = 128; the dQ
+// kernel keeps the iterative-ILP scheduler, which measured 2-5% faster for it.
 #include <algorithm>
 
 #include "attn_common.h"
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   static_assert(PRE >= 2 && PRE < NBUF, "tiles 0 and 1 are in flight before the loop");
   static_assert(NBUF >= 4, "a barrier every second tile needs two tiles of slack");
   static_assert(NBUF * PER < 64 && 2 * NS + 2 * NCH + PRE * PER < 64, "vmcnt range");
-  __shared__ __attribute__((aligned(1024))) char ring[NBUF * SLOTB];
+  __shared__ __attribute__((aligned(4096))) char ring[NBUF * SLOTB];
   __shared__ __attribute__((aligned(256))) float stbuf[NBUF][128];  // [0, 64): -lse * log2(e), [64, 128): -delta
 
   const int T = a.T, W = a.W, H = a.H, Hkv = a.Hkv;
@@ -166,21 +166,19 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   // 3. Wait for this wave's K and V rows (the first tiles may be in flight).
   vm_wait_upto<PER, PRE>(n_pre);
 
-  // Operand offsets: kept in registers for D = 64, recomputed per use for
-  // D = 128 (whose accumulators leave no room for them).
+  // Operand offsets: kept in registers for D = 64; D = 128, whose accumulators
+  // leave no room for them, keeps one of each kind and forms the others from
+  // it by XOR (valid with the ring's base included: the ring is 4 KB aligned
+  // and the XORed bits lie below that).
   constexpr bool KEEP_TRO = D == 64;
-  const int rbase = (l32 / L::RPC) * 1024 + (l32 % L::RPC) * L::U * 16, fr = L::f(l32);
   int off_s[NS];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) off_s[s] = KEEP_TRO ? L::byte(l32, 2 * s + h32) : 0;
-  auto offs = [&](int s) __attribute__((always_inline)) {
-    return KEEP_TRO ? off_s[s] : rbase + (((2 * s + h32) ^ fr) << 4);
-  };
+  for (int s = 0; s < NS; ++s) off_s[s] = L::byte(l32, 2 * s + h32);
   int tro[NDB][2];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) {
-    tro[db][0] = KEEP_TRO ? cs_tr_off<D>(db, 0, lane) : 0;
-    tro[db][1] = KEEP_TRO ? cs_tr_off<D>(db, 1, lane) : 0;
+    tro[db][0] = cs_tr_off<D>(db, 0, lane);
+    tro[db][1] = cs_tr_off<D>(db, 1, lane);
   }
   // K^T (times scale * log2(e)) and V^T as B operands: lane l holds row
   // kw0 + l % 32, columns 16 s + 8 (l / 32) + e.
@@ -188,8 +186,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     if constexpr (STAGE_KV) {
-      kraw[s] = cs_operand<D>(stg_k, offs(s), 0);
-      vraw[s] = cs_operand<D>(stg_v, offs(s), 0);
+      kraw[s] = cs_operand<D>(stg_k, off_s[s], 0);
+      vraw[s] = cs_operand<D>(stg_v, off_s[s], 0);
     }
     kreg[s] = scale_bf16x8(kraw[s], c);
     vreg[s] = vraw[s];
@@ -239,7 +237,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
         asm volatile("" : "+v"(atr[db][k]));
       }
   }
-  const unsigned lbase = KEEP_TRO ? 0u : lring;  // the part of the ring address not in ab_s / atr
+  const unsigned ab0 = lring + (unsigned)off_s[0], at00 = lring + (unsigned)tro[0][0];
 
   for (int it0 = 0; it0 < n_iter; it0 += NBUF)
 #pragma unroll
@@ -268,7 +266,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
       }
     }
 
-    const unsigned qs_t = lbase + (unsigned)slot * SLOTB, ds_t = qs_t + TILEB;
+    const unsigned qs_t = (unsigned)slot * SLOTB, ds_t = qs_t + TILEB;  // constants; the base is in the offsets
     const float* st = stbuf[slot];
     const int qs = (tq_lo + qtile_of(cp_t)) * BMQ;
     if (++cp_t == nq) cp_t = 0;
@@ -300,20 +298,29 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
     }
 
     f32x16 sacc = si, pacc = di;
-    if constexpr (D == 64) __builtin_amdgcn_sched_barrier(0);
+    // D = 128: the XOR variants are formed per tile from copies made opaque
+    // here, so they are not hoisted into 16 registers of their own.
+    unsigned ab = ab0, tb = at00;
+    if constexpr (!KEEP_TRO) asm volatile("" : "+v"(ab), "+v"(tb));
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const int o = KEEP_TRO ? (int)ab_s[s] : offs(s);
+      const int o = KEEP_TRO ? (int)ab_s[s] : (int)(ab ^ (32u * s));
       sacc = mfma32(cs_operand<D>(qs_t, o, 0), kreg[s], sacc);
       pacc = mfma32(cs_operand<D>(ds_t, o, 0), vreg[s], pacc);
     }
-    if constexpr (D == 64) {
-      // The 8 row-operand reads run two ahead of their products (a ds_read,
-      // then alternately one MFMA and the next read): left to itself the
-      // scheduler issued each read right before its product and waited for
-      // it there, so every S and dP product waited out a full LDS latency.
-      // Two operand buffers fit in the 168 VGPRs of three waves per SIMD.
-      constexpr int AHEAD = 2;
+    {
+      // The row-operand reads run ahead of their products (some ds_reads, then
+      // alternately one MFMA and the next read): left to itself the scheduler
+      // issued each read right before its product and waited for it there, so
+      // every S and dP product waited out a full LDS latency.  Two operand
+      // buffers fit in the 168 VGPRs of three waves per SIMD (D = 64), three in
+      // the 256 of two (D = 128, where the transposed reads of dV and dK below
+      // run three ahead too).  D = 128, before and after: T = 1777 on 112
+      // workgroups 205 -> 158 us, 3 x 1000 W = 300 23.6 -> 20.1, 4 x 4096 W = 1024
+      // 182.4 -> 171.9, causal 368 -> 350, 16384 W = 2048 448 -> 446 (two ahead
+      // 172.5 / 346 / 447, four 174 / 353 / 449).
+      constexpr int AHEAD = D == 64 ? 2 : 3;
       __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);  // DS reads
 #pragma unroll
       for (int i = 0; i < 2 * NS - AHEAD; ++i) {
@@ -334,11 +341,22 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
       for (int db = 0; db < NDB; ++db) {
-        const int o0 = KEEP_TRO ? (int)atr[db][0] : cs_tr_off<D>(db, 0, lane);
-        const int o1 = KEEP_TRO ? (int)atr[db][1] : cs_tr_off<D>(db, 1, lane);
+        const int o0 = KEEP_TRO ? (int)atr[db][0] : cs_tr_off_from<D>((int)tb, db, 0);
+        const int o1 = KEEP_TRO ? (int)atr[db][1] : cs_tr_off_from<D>((int)tb, db, 1);
         dvacc[db] = mfma32(cs_operand_tr<D>(ds_t, o0, o1, 16 * kk), pb[kk], dvacc[db]);
         dkacc[db] = mfma32(cs_operand_tr<D>(qs_t, o0, o1, 16 * kk), dsb[kk], dkacc[db]);
       }
+    if constexpr (D == 128) {  // (at D = 64 this order measured 0-1% slower)
+      constexpr int AHEAD = 3;  // transposed operands, two reads each
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * AHEAD, 0);
+#pragma unroll
+      for (int i = 0; i < 4 * NDB - AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 
   if constexpr (SPLIT) {
@@ -452,20 +470,23 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_merge_kernel(BwdArgs a
 
 // The chunks of a split dK/dV for these sizes; n = 0 where it does not pay.
 //
-// A key tile's workgroup walks its query tiles one after the other: 1.2 us
-// each at D = 128 and 0.65 us at D = 64 while workgroups have a CU to
+// A key tile's workgroup walks its query tiles one after the other: 0.93 us
+// each at D = 128 and 0.62 us at D = 64 while workgroups have a CU to
 // themselves, so a grid that does not fill the chip takes as long as its
 // longest key tile.  In chunks that fill the workgroup slots once, a query
-// tile takes about 1.5 (D = 128) or 2.5 (D = 64) times that, beside about
-// 8 us for the second prologue, the fp32 partial sums and the merge: the
-// comparison below, in query tiles.  Chunks that fill the slots one and a
-// half or two times, or half, measured slower (B = 2, T = 1777, 12 query on 4
-// kv heads, D = 128, causal: backward 253 us unsplit, 111 us at one filling,
-// 133 / 131 / 126 at 1.5, 2 and 0.5).  Others, backward before and after: B = 1,
-// T = 2048, H = 6, D = 64, causal 71.6 -> 52.6 us; 12 on 4 heads, W = 512
-// 52.5 -> 35.0; 8 on 1, T = 8192 1289 -> 308; T = 8192, 16 on 4, D = 128,
-// W = 2048 504 -> 415; T = 1777, 12 on 12, D = 128 124 -> 112.  Where the rule says no: T = 4096, H = 16, D = 64, causal
-// 154.8 against 159.5 us split.
+// tile takes about 1.5 (D = 128) or 2.5 (D = 64) times that, beside the second
+// prologue, the fp32 partial sums and the merge (26 query tiles' time at D =
+// 128 where 512 chunks write sums, 12 at D = 64): the comparisons below, in
+// query tiles.  Chunks that fill the slots one and a half or two times, or
+// half, measured slower (B = 2, T = 1777, 12 query on 4 kv heads, D = 128,
+// causal: 20% at 1.5 and 2, 12% at 0.5).
+//
+// dK/dV with its merge, us, unsplit and split.  D = 128, causal unless W is
+// given: that shape 155 / 60; 12 on 12 heads 58 / 60 (refused); T = 8192, 16 on
+// 4, W = 2048 251 / 227; T = 2048, 12 heads 62 / 47; T = 1536, 16 heads 48 / 42;
+// T = 4096, 8 heads, W = 1024 38 / 51 (refused).  D = 64: T = 2048, 6 heads
+// 40 / 21; T = 4096, 12 heads 80 / 69; 2 x 2048, 12 heads 43 / 44 (refused);
+// T = 8192, 8 on 1 head 1157 / 180.
 DkdvSplit dkdv_split_plan(int B, int T, int H, int Hkv, int D, int W) {
   constexpr int64_t kMinLen = 16;
   DkdvSplit s{};
@@ -483,12 +504,14 @@ DkdvSplit dkdv_split_plan(int B, int T, int H, int Hkv, int D, int W) {
   int64_t total = 0;
   for (int kt = 0; kt < nkt; ++kt) total += len(kt);
   int64_t c = std::max({(total * units + slots - 1) / slots, (longest + kMaxDkdvChunks - 1) / kMaxDkdvChunks, kMinLen});
+  int64_t blocks = 0;
   for (; c < longest; c += std::max(c / 32, (int64_t)1)) {
-    int64_t blocks = 0;
+    blocks = 0;
     for (int kt = 0; kt < nkt; ++kt) blocks += (len(kt) + c - 1) / c;
-    if (blocks * units <= slots) break;
+    blocks *= units;
+    if (blocks <= slots) break;
   }
-  if (D == 64 ? 5 * c + 24 >= 2 * longest : 3 * c + 16 >= 2 * longest) return s;
+  if (D == 64 ? 5 * c + 24 >= 2 * longest : 3 * c + 12 + 5 * blocks / 64 >= 2 * longest) return s;
   s.len = (int)c;
   for (; s.n * c < longest; ++s.n) {
     int has = 0;  // key tiles with a chunk s.n

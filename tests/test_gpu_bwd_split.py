@@ -54,6 +54,7 @@ def test_split_applies_to_the_cases_below(case):
         (1, 1000, 6, 6, 64, 300),      # short rows
         (1, 333, 4, 1, 64, 129),
         (1, 4096, 16, 16, 64, None),   # chunks would be as long as the slots they fill are slow
+        (1, 4096, 8, 8, 128, 1024),
         (0, 128, 2, 2, 64, None),
     ],
 )
