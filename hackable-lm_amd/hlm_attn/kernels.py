@@ -249,13 +249,13 @@ class _LMHeadLoss(torch.autograd.Function):
 
     The rows are processed in chunks (`linear_ce_chunk_size`).  One logits
     workspace of chunk x V is allocated once and every chunk's GEMM writes
-    into it; the HIP row kernel (hackable_lm::hip_linear_ce) turns it in
-    place into the gradient of the mean loss and returns the rows' losses.
+    into it; the HIP row kernel (hackable_lm::hip_linear_ce_into) turns it in
+    place into the gradient of the mean loss and writes the rows' losses.
     The three gradient products are formed in the forward, straight into
     their destinations: dhidden rows by a GEMM whose output is the chunk's
     slice of the dhidden buffer (hackable_lm::hip_ce_dhidden where it beats the
-    library's), dW accumulated inside the GEMM (addmm_, one
-    rounding per chunk), db by an in-place add.  The backward only scales the
+    library's), dW written by the first chunk's GEMM and accumulated inside the
+    others' (addmm_, one rounding per chunk), db by an in-place add.  The backward only scales the
     three by the incoming gradient.  The results match the reference's
     chunked loop (kernels.py:878-942), which this replaces."""
 
@@ -272,7 +272,7 @@ class _LMHeadLoss(torch.autograd.Function):
         want_h, want_w = hidden.requires_grad, weight.requires_grad
         want_b = bias is not None and bias.requires_grad
         d_hidden = torch.empty_like(hidden) if want_h else None
-        d_weight = torch.zeros_like(weight) if want_w else None
+        d_weight = torch.empty_like(weight) if want_w else None
         d_bias = torch.zeros_like(bias) if want_b else None
         losses = torch.empty(n, dtype=torch.float32, device=hidden.device)
         # Rows of the workspace start on 128-byte lines: with V = 50257 the three
@@ -294,10 +294,12 @@ class _LMHeadLoss(torch.autograd.Function):
                 torch.mm(h, w_t, out=g)
             else:
                 torch.addmm(bias, h, w_t, out=g)
-            losses[r0:r1] = ops.hip_linear_ce(g, targets[r0:r1], n)
+            ops.hip_linear_ce_into(g, targets[r0:r1], n, losses[r0:r1])
             if want_h:
                 ops.hip_ce_dhidden(padded[: r1 - r0], weight, vocab, d_hidden[r0:r1])
-            if want_w:
+            if want_w and r0 == 0:
+                torch.mm(g.t(), h, out=d_weight)
+            elif want_w:
                 d_weight.addmm_(g.t(), h)
             if want_b:
                 d_bias.add_(g.sum(dim=0).to(d_bias.dtype))
@@ -306,15 +308,17 @@ class _LMHeadLoss(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        d_hidden, d_weight, d_bias = ctx.saved_tensors
-        out = []
-        for need, t in ((ctx.needs_input_grad[0], d_hidden), (ctx.needs_input_grad[1], d_weight)):
-            out.append(t * grad_output.to(t.dtype) if need and t is not None else None)
-        out.append(None)
-        need_b = ctx.needs_input_grad[3] and d_bias is not None
-        out.append(d_bias * grad_output.to(d_bias.dtype) if need_b else None)
-        out.append(None)
-        return tuple(out)
+        grads = []
+        scale = grad_output  # in the gradients' type, converted once
+        for i, t in zip((0, 1, 3), ctx.saved_tensors):
+            if t is None or not ctx.needs_input_grad[i]:
+                grads.append(None)
+                continue
+            if scale.dtype != t.dtype:
+                scale = grad_output.to(t.dtype)
+            grads.append(t * scale)
+        d_hidden, d_weight, d_bias = grads
+        return d_hidden, d_weight, None, d_bias, None
 
 
 def fused_linear_cross_entropy_with_weight(

@@ -448,8 +448,8 @@ hip_qk_norm_rope.register_autograd(_qk_backward, setup_context=_qk_setup_context
 IGNORE_INDEX = -100  # F.cross_entropy's default ignore_index
 
 
-def linear_ce_impl(logits: torch.Tensor, targets: torch.Tensor, n_tokens: int) -> torch.Tensor:
-    """The launch behind hackable_lm::hip_linear_ce."""
+def linear_ce_impl(logits: torch.Tensor, targets: torch.Tensor, n_tokens: int, loss: torch.Tensor | None = None) -> torch.Tensor:
+    """The launch behind hackable_lm::hip_linear_ce, into `loss` if given."""
     if logits.device.type != "cuda":
         raise RuntimeError(f"hip linear_ce runs on ROCm devices only, got a tensor on {logits.device}")
     if logits.dim() != 2 or logits.stride(1) != 1:
@@ -460,7 +460,10 @@ def linear_ce_impl(logits: torch.Tensor, targets: torch.Tensor, n_tokens: int) -
         raise RuntimeError(f"targets {tuple(targets.shape)} do not match {logits.shape[0]} logit rows")
     lib = _lib.load()
     targets = targets.to(device=logits.device, dtype=torch.int64).contiguous()
-    loss = torch.empty(logits.shape[0], dtype=torch.float32, device=logits.device)
+    if loss is None:
+        loss = torch.empty(logits.shape[0], dtype=torch.float32, device=logits.device)
+    elif loss.shape != targets.shape or loss.dtype != torch.float32 or loss.device != logits.device or not loss.is_contiguous():
+        raise RuntimeError(f"hip linear_ce expects a contiguous float32 loss of {logits.shape[0]} rows")
     code = _lib.DTYPE_BF16 if logits.dtype == _BF16 else _lib.DTYPE_F32
     with _on_device(logits.device):
         rc = lib.hlm_ce_rows(
@@ -479,6 +482,17 @@ def hip_linear_ce(logits: torch.Tensor, targets: torch.Tensor, n_tokens: int) ->
 @hip_linear_ce.register_fake
 def _(logits, targets, n_tokens):
     return logits.new_empty((logits.shape[0],), dtype=torch.float32)
+
+
+@torch.library.custom_op("hackable_lm::hip_linear_ce_into", mutates_args=("logits", "loss"))
+def hip_linear_ce_into(logits: torch.Tensor, targets: torch.Tensor, n_tokens: int, loss: torch.Tensor) -> None:
+    """hip_linear_ce with the rows' losses written to `loss`."""
+    linear_ce_impl(logits, targets, n_tokens, loss)
+
+
+@hip_linear_ce_into.register_fake
+def _(logits, targets, n_tokens, loss):
+    return None
 
 
 def _ce_dhidden_ready(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> bool:
