@@ -18,6 +18,8 @@
 //                         can see its keys, accumulating dK and dV in VGPRs
 //                         (attn_bwd_dkdv.hip, compiled with another scheduler).
 // Both skip whole tiles outside the causal window, so cost scales with T * W.
+// Where a grid of whole tiles would leave the chip idle, a tile's walk is cut
+// into chunks that a merge kernel sums (dq_chunk_plan, dkdv_chunk_plan).
 //
 // Per score element the VALU does two operations (exp2, multiply) plus two
 // half bf16 conversions:
@@ -65,7 +67,7 @@ __device__ __forceinline__ f32x16 splat16(float v) {
 // them, and no store is issued before the loop ends, so inside the loop the
 // vector-memory counter counts tile copies only.
 // ---------------------------------------------------------------------------
-template <int D, int NBUF, int PRE>
+template <int D, int NBUF, int PRE, bool SPLIT>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(BwdArgs a) {
   using L = CS<D>;
   constexpr int NW = 4, BM = NW * 32, BN = 32;
@@ -84,7 +86,14 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(BwdAr
 
   const int T = a.T, W = a.W, H = a.H;
   const int nqt = (T + BM - 1) / BM;
-  const TileId tid_ = tile_order(blockIdx.x, a.B * H, nqt - (W - 1 + BM - 1) / BM);
+  TileId tid_ = SPLIT ? rank_major(blockIdx.x, a.B * H) : tile_order(blockIdx.x, a.B * H, nqt - (W - 1 + BM - 1) / BM);
+  int chunk = 0;
+  if constexpr (SPLIT) {
+    // Ranks run over chunk 0 of every query tile, then chunk 1 of those that
+    // have one, ...
+    while (chunk + 1 < a.qchunks.n && tid_.rank >= a.qchunks.base[chunk + 1]) ++chunk;
+    tid_.rank -= a.qchunks.base[chunk];
+  }
   const int qt = nqt - 1 - tid_.rank;  // longest causal rows first
   const int bh = tid_.unit;
   const int h = bh % H, b = bh / H;
@@ -93,6 +102,24 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(BwdAr
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, h32 = lane >> 5;
   const int q0 = qt * BM, qw0 = q0 + 32 * wave, myq = qw0 + l32;
+
+  // The partial sums of a query tile of several chunks, in the accumulators'
+  // order ([wave][db][i][lane] x 4 floats).
+  const bool cut = SPLIT && tid_.rank < a.qchunks.base[2] - a.qchunks.base[1];
+  auto part_of = [&](int ln) __attribute__((always_inline)) {
+    return reinterpret_cast<f32x4*>(a.qchunks.part) +
+           ((int64_t)(a.qchunks.base[chunk] + tid_.rank) * (a.B * H) + bh) * (BM * D / 4) + wave * (NDB * 4 * 64) + ln;
+  };
+  if constexpr (SPLIT) {
+    // A ragged last query tile may meet up to three key tiles less than the one
+    // before it and then lack the last chunk.
+    if (cut && chunk * a.qchunks.len > (min(T, q0 + BM) - 1) / BN - max(0, q0 - W + 1) / BN) {
+      f32x4* part = part_of(lane);
+#pragma unroll
+      for (int x = 0; x < NDB * 4; ++x) part[x * 64] = f32x4{0.f, 0.f, 0.f, 0.f};
+      return;
+    }
+  }
 
   const __amdgpu_buffer_rsrc_t rq = slab_rsrc(a.q + b * a.sq[0] + h * a.sq[2], a.sq[1], T, D);
   const __amdgpu_buffer_rsrc_t rdo = slab_rsrc(a.dout + b * a.sdo[0] + h * a.sdo[2], a.sdo[1], T, D);
@@ -117,11 +144,15 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(BwdAr
   // 2. The first ring tiles.
   const int key_lo = max(0, q0 - W + 1);
   const int key_hi = min(T, q0 + BM) - 1;
-  const int t_lo = key_lo / BN, n_tiles = key_hi / BN - t_lo + 1;
+  int t_lo = key_lo / BN, n_tiles = key_hi / BN - t_lo + 1;
+  if constexpr (SPLIT) {
+    t_lo += chunk * a.qchunks.len;
+    n_tiles = min(a.qchunks.len, n_tiles - chunk * a.qchunks.len);
+  }
   // Key tiles in the forward's rotated order (step t reads the tile congruent
   // to t modulo n_tiles), so that the workgroups on one XCD, whose windows
   // are offset by a few tiles each, read the same K/V tiles at the same step.
-  const int rot = (n_tiles - t_lo % n_tiles) % n_tiles;
+  const int rot = SPLIT ? 0 : (n_tiles - t_lo % n_tiles) % n_tiles;
   auto tile_of = [&](int t) __attribute__((always_inline)) {
     const int g = t + rot;
     return t_lo + (g >= n_tiles ? g - n_tiles : g);
@@ -374,6 +405,29 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(BwdAr
     }
   }
 
+  if constexpr (SPLIT) {
+    if (chunk == 0 && myq < T && h32 == 0) {
+      a.delta[(int64_t)bh * T + myq] = nlse2;
+      a.delta[(int64_t)(a.B * H + bh) * T + myq] = ndelta;
+    }
+    if (cut) {
+      // (Every issued tile has been waited for inside the loop.)
+      int ln = lane;
+      asm volatile("" : "+v"(ln));  // the address is computed here, not kept over the loop
+      f32x4* part = part_of(ln);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f32x4 v4;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v4[j] = dqacc[db][4 * i + j];
+          part[(db * 4 + i) * 64] = v4;
+        }
+      return;
+    }
+  }
+
   // dQ through LDS: every wave is past its last tile, so wave w may use the
   // bytes [32 rows * w, 32 rows * (w + 1)) of the ring for its block.
   dma_barrier<0>();
@@ -401,10 +455,60 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_bwd_dq_kernel(BwdAr
     bf16x8* dst = reinterpret_cast<bf16x8*>(dqbase + (int64_t)(qw0 + row) * a.sdq[1] + 8 * (ln % L::U));
     if (qw0 + row < T) __builtin_nontemporal_store(v, dst);
   }
-  if (myq < T && h32 == 0) {
+  if (!SPLIT && myq < T && h32 == 0) {
     a.delta[(int64_t)bh * T + myq] = nlse2;
     a.delta[(int64_t)(a.B * H + bh) * T + myq] = ndelta;
   }
+}
+
+// Sums the chunks of a split dQ: one workgroup per 32 queries of one (batch,
+// head).
+template <int D>
+__global__ __launch_bounds__(kThreads) void attn_bwd_dq_merge_kernel(BwdArgs a) {
+  constexpr int64_t BLOCK = 128 * D / 4;  // f32x4 of a chunk
+  __shared__ __attribute__((aligned(1024))) char rows[32 * D * 2];
+  const int units = a.B * a.H, quarter = blockIdx.x & 3;
+  const int rank = (int)(blockIdx.x >> 2) / units, unit = (int)(blockIdx.x >> 2) % units;
+  const int h = unit % a.H, b = unit / a.H, qt = (a.T + 127) / 128 - 1 - rank;
+  int n = 0;  // chunks of this query tile
+  while (n < a.qchunks.n && rank < a.qchunks.base[n + 1] - a.qchunks.base[n]) ++n;
+  const f32x4* src = reinterpret_cast<const f32x4*>(a.qchunks.part) + quarter * (BLOCK / 4);
+  auto block = [&](int c) __attribute__((always_inline)) {
+    return src + ((int64_t)(a.qchunks.base[c] + rank) * units + unit) * BLOCK;
+  };
+  sum_chunk_rows<D>(n, block, a.scale, a.dq + b * a.sdq[0] + h * a.sdq[2], a.sdq[1], qt * 128 + quarter * 32, a.T,
+                    lds_addr(rows));
+}
+
+// The chunks of a split dQ for these sizes; n = 0 where it does not pay.
+//
+// A query tile's workgroup walks its key tiles one after the other, so a grid
+// that leaves slots empty takes as long as its longest tile (D = 64: 0.9 of a
+// microsecond for two key tiles, D = 128: 0.85 for one) however much of the
+// chip is idle.  Chunks fill the slots, but two or three resident workgroups a
+// CU slow each other down, and a cut tile pays a store of its sums and the
+// merge pass.  Fitted over 30 shapes, splitting pays while
+//   D = 64:  2 chunk + chunk blocks / 400 + blocks / 18 + 15 < 2 longest
+//   D = 128: 2 chunk + 5 blocks / 64 + 12 < 2 longest   (in key tiles of 32)
+// Whole backward with dQ unsplit -> split (us), causal unless W is given:
+//   taken    D = 64:  2048x12 60 -> 51, 4096x4 94 -> 64, 8000x4 188 -> 142, 4096x12 131 -> 124,
+//                     1500x4 55 -> 47, 1000x6 40 -> 38, 2x1500x8 56 -> 55, 2000x4 W 1024 45 -> 42
+//            D = 128: 2048x12 101 -> 84, 8000x4 335 -> 257, 2x1777x12 112 -> 108, 1024x16 64 -> 61
+//   refused  D = 64:  2x2048x16 88 -> 93, 3000x8 W 1024 45 -> 50, 2x2048x12 76 -> 76
+//            D = 128: 2048x16 W 512 48 -> 55, 4096x8 W 1024 73 -> 78, 2x1500x8 W 700 59 -> 61
+// Chunks of 16 and 24 key tiles at the least came out the same but for short
+// rows (2048x6 at D = 64: 39 and 41; 1024x16 at D = 128: 61 and 64).
+ChunkPlan dq_chunk_plan(int B, int T, int H, int D, int W) {
+  const int nqt = (T + 127) / 128;
+  // Key tiles that the query tile of rank r meets.
+  auto len = [=](int r) {
+    const int64_t q0 = (int64_t)(nqt - 1 - r) * 128;
+    return (std::min<int64_t>(T, q0 + 128) - 1) / 32 - std::max<int64_t>(0, q0 - W + 1) / 32 + 1;
+  };
+  auto pays = [=](int64_t c, int64_t blocks, int64_t longest) {
+    return (D == 64 ? 2 * c + c * blocks / 400 + blocks / 18 + 15 : 2 * c + 5 * blocks / 64 + 12) < 2 * longest;
+  };
+  return plan_chunks(len, nqt, (int64_t)B * H, 256 * (D == 64 ? 3 : 2), 16, pays);
 }
 
 // attn_bwd_dkdv.hip
@@ -416,13 +520,20 @@ hipError_t launch_bwd(const BwdArgs& a, hipStream_t stream, int phases) {
   if (phases & kBwdDq) {
     constexpr int BM = 128;
     const int nqt = (a.T + BM - 1) / BM;
-    const int64_t blocks = (int64_t)nqt * a.H * a.B;
+    const int64_t units = (int64_t)a.H * a.B;
     // D = 64: 6 slots of 8 KB, two tiles in flight while the staging (4 slots) is used;
     // D = 128: 5 slots of 16 KB, one tile in flight.
-    if constexpr (D == 64)
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, 6, 2>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
-    else
-      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, 5, 1>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+    constexpr int NBUF = D == 64 ? 6 : 5, PRE = D == 64 ? 2 : 1;
+    if (a.qchunks.n == 0) {
+      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NBUF, PRE, false>), dim3((unsigned)(nqt * units)), dim3(256), 0, stream, a);
+    } else {
+      hipLaunchKernelGGL((attn_bwd_dq_kernel<D, NBUF, PRE, true>), dim3((unsigned)(a.qchunks.base[a.qchunks.n] * units)),
+                         dim3(256), 0, stream, a);
+      const hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return err;
+      const int64_t cut = a.qchunks.base[2] - a.qchunks.base[1];
+      hipLaunchKernelGGL((attn_bwd_dq_merge_kernel<D>), dim3((unsigned)(cut * units * 4)), dim3(kThreads), 0, stream, a);
+    }
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }

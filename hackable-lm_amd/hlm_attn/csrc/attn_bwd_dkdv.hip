@@ -6,8 +6,6 @@
 // scheduler, which honours the sched_group_barrier pipelines of the operand
 // reads below within three waves per SIMD at D = 64 and two at D = 128; the dQ
 // kernel keeps the iterative-ILP scheduler, which measured 2-5% faster for it.
-#include <algorithm>
-
 #include "attn_common.h"
 
 namespace hlm {
@@ -57,8 +55,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   if constexpr (SPLIT) {
     // Ranks run over chunk 0 of every key tile, then chunk 1 of those that
     // have one, ...
-    while (chunk + 1 < a.split.n && kt >= a.split.base[chunk + 1]) ++chunk;
-    kt -= a.split.base[chunk];
+    while (chunk + 1 < a.kchunks.n && kt >= a.kchunks.base[chunk + 1]) ++chunk;
+    kt -= a.kchunks.base[chunk];
   }
   const int bhk = tid_.unit;
   const int hk = bhk % Hkv, b = bhk / Hkv;
@@ -73,8 +71,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   const int tq_lo = q_lo / BMQ, tq_hi = q_hi / BMQ;
   const int nq = tq_hi - tq_lo + 1;
   // The query tiles this workgroup visits, of the nq * G of its key tile.
-  const int it_lo = SPLIT ? chunk * a.split.len : 0;
-  const int n_iter = SPLIT ? min(a.split.len, nq * G - it_lo) : nq * G;
+  const int it_lo = SPLIT ? chunk * a.kchunks.len : 0;
+  const int n_iter = SPLIT ? min(a.kchunks.len, nq * G - it_lo) : nq * G;
   const int sq2 = (int)(a.sq[1] * 2), sdo2 = (int)(a.sdo[1] * 2);
 
   // Start values: waves 0 and 2 copy a tile's -lse*log2(e) row, waves 1 and 3
@@ -360,12 +358,12 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   }
 
   if constexpr (SPLIT) {
-    if (kt < a.split.base[2] - a.split.base[1]) {
+    if (kt < a.kchunks.base[2] - a.kchunks.base[1]) {
       // The key tile has more chunks: fp32 partial sums, in the accumulators'
       // own order ([wave][dK, dV][db][i][lane] x 4 floats, 1 KB a store).
       // Every issued tile has been waited for inside the loop.
-      f32x4* dst = reinterpret_cast<f32x4*>(a.split.part) +
-                   ((int64_t)(a.split.base[chunk] + kt) * (a.B * Hkv) + bhk) * (BNK * D / 2) + wave * (2 * NDB * 4 * 64) + lane;
+      f32x4* dst = reinterpret_cast<f32x4*>(a.kchunks.part) +
+                   ((int64_t)(a.kchunks.base[chunk] + kt) * (a.B * Hkv) + bhk) * (BNK * D / 2) + wave * (2 * NDB * 4 * 64) + lane;
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -419,53 +417,24 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   }
 }
 
-// Sums the chunks of a split dK/dV in their order and writes bf16 rows;
-// bound by reading the partial sums once, fully coalesced.  One
-// workgroup per 32 keys of one (batch, kv head) and one of dK, dV: thread
-// (lane, wave) adds the f32x4 pieces piece = wave, wave + 4, ... of the
-// block, and the rows leave through LDS.
+// Sums the chunks of a split dK/dV: one workgroup per 32 keys of one (batch,
+// kv head) and one of dK, dV.
 template <int D>
 __global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_merge_kernel(BwdArgs a) {
-  using L = CS<D>;
-  constexpr int NDB = D / 32, PIECES = NDB * 4, PPT = PIECES / 4;  // f32x4 per thread and chunk
-  constexpr int64_t BLOCK = 128 * D / 2;                          // f32x4 per chunk block (dK and dV)
+  constexpr int64_t BLOCK = 128 * D / 2, ROWS = 32 * D / 4;  // f32x4 of a chunk (dK and dV), of 32 rows of one
   __shared__ __attribute__((aligned(1024))) char rows[32 * D * 2];
-  const int units = a.B * a.Hkv, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int which = blockIdx.x & 1, quarter = (blockIdx.x >> 1) & 3;
+  const int units = a.B * a.Hkv, which = blockIdx.x & 1, quarter = (blockIdx.x >> 1) & 3;
   const int kt = (int)(blockIdx.x >> 3) / units, unit = (int)(blockIdx.x >> 3) % units;
+  const int hk = unit % a.Hkv, b = unit / a.Hkv;
   int n = 0;  // chunks of this key tile
-  while (n < a.split.n && kt < a.split.base[n + 1] - a.split.base[n]) ++n;
-  f32x4 acc[PPT];
-#pragma unroll
-  for (int p = 0; p < PPT; ++p) acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const f32x4* src = reinterpret_cast<const f32x4*>(a.split.part) + quarter * (2 * PIECES * 64) + which * (PIECES * 64) +
-                     wave * 64 + lane;
-  for (int c = 0; c < n; ++c) {
-    const f32x4* s = src + ((int64_t)(a.split.base[c] + kt) * units + unit) * BLOCK;
-#pragma unroll
-    for (int p = 0; p < PPT; ++p) acc[p] += s[p * 256];
-  }
-  const float f = which == 0 ? a.scale : 1.f;
-  const unsigned base = lds_addr(rows);
-#pragma unroll
-  for (int p = 0; p < PPT; ++p) {
-    const int piece = wave + 4 * p;  // 4 db + i
-    bf16x4 v;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = (bf16)(acc[p][j] * f);
-    lds_write_b64(base + L::byte(lane & 31, piece) + 8 * (lane >> 5), v);
-  }
-  __syncthreads();
-  const int hk = unit % a.Hkv, b = unit / a.Hkv, row0 = kt * 128 + quarter * 32;
+  while (n < a.kchunks.n && kt < a.kchunks.base[n + 1] - a.kchunks.base[n]) ++n;
+  const f32x4* src = reinterpret_cast<const f32x4*>(a.kchunks.part) + (2 * quarter + which) * ROWS;
+  auto block = [&](int c) __attribute__((always_inline)) {
+    return src + ((int64_t)(a.kchunks.base[c] + kt) * units + unit) * BLOCK;
+  };
   const int64_t* st = which == 0 ? a.sdk : a.sdv;
-  bf16* dst = (which == 0 ? a.dk : a.dv) + b * st[0] + hk * st[2];
-#pragma unroll
-  for (int k = 0; k < 32 * L::U / 256; ++k) {
-    const int row = (tid + 256 * k) / L::U, u = tid % L::U;
-    if (row0 + row < a.T)
-      __builtin_nontemporal_store(lds_read_b128(base + L::byte(row, u)),
-                                  reinterpret_cast<bf16x8*>(dst + (int64_t)(row0 + row) * st[1] + 8 * u));
-  }
+  sum_chunk_rows<D>(n, block, which == 0 ? a.scale : 1.f, (which == 0 ? a.dk : a.dv) + b * st[0] + hk * st[2], st[1],
+                    kt * 128 + quarter * 32, a.T, lds_addr(rows));
 }
 
 // The chunks of a split dK/dV for these sizes; n = 0 where it does not pay.
@@ -487,38 +456,17 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_merge_kernel(BwdArgs a
 // T = 4096, 8 heads, W = 1024 38 / 51 (refused).  D = 64: T = 2048, 6 heads
 // 40 / 21; T = 4096, 12 heads 80 / 69; 2 x 2048, 12 heads 43 / 44 (refused);
 // T = 8192, 8 on 1 head 1157 / 180.
-DkdvSplit dkdv_split_plan(int B, int T, int H, int Hkv, int D, int W) {
-  constexpr int64_t kMinLen = 16;
-  DkdvSplit s{};
-  const int slots = 256 * (D == 64 ? 3 : 2), G = H / Hkv;
-  const int64_t units = (int64_t)B * Hkv, tiles = ((int64_t)T + 127) / 128;
-  if (units * tiles >= slots) return s;
-  const int nkt = (int)tiles;
-  // Query tiles that key tile kt meets, over the group's heads (never more
-  // than for the key tile before it).
-  auto len = [&](int kt) {
-    const int k0 = kt * 128;
-    return (std::min((int64_t)T - 1, (int64_t)k0 + 126 + W) / 32 - k0 / 32 + 1) * G;
+ChunkPlan dkdv_chunk_plan(int B, int T, int H, int Hkv, int D, int W) {
+  const int G = H / Hkv;
+  // Query tiles that a key tile meets, over the group's heads.
+  auto len = [=](int kt) {
+    const int64_t k0 = kt * 128;
+    return (std::min<int64_t>(T - 1, k0 + 126 + W) / 32 - k0 / 32 + 1) * G;
   };
-  const int64_t longest = len(0);
-  int64_t total = 0;
-  for (int kt = 0; kt < nkt; ++kt) total += len(kt);
-  int64_t c = std::max({(total * units + slots - 1) / slots, (longest + kMaxDkdvChunks - 1) / kMaxDkdvChunks, kMinLen});
-  int64_t blocks = 0;
-  for (; c < longest; c += std::max(c / 32, (int64_t)1)) {
-    blocks = 0;
-    for (int kt = 0; kt < nkt; ++kt) blocks += (len(kt) + c - 1) / c;
-    blocks *= units;
-    if (blocks <= slots) break;
-  }
-  if (D == 64 ? 5 * c + 24 >= 2 * longest : 3 * c + 12 + 5 * blocks / 64 >= 2 * longest) return s;
-  s.len = (int)c;
-  for (; s.n * c < longest; ++s.n) {
-    int has = 0;  // key tiles with a chunk s.n
-    while (has < nkt && len(has) > s.n * c) ++has;
-    s.base[s.n + 1] = s.base[s.n] + has;
-  }
-  return s;
+  auto pays = [=](int64_t c, int64_t blocks, int64_t longest) {
+    return D == 64 ? 5 * c + 24 < 2 * longest : 3 * c + 12 + 5 * blocks / 64 < 2 * longest;
+  };
+  return plan_chunks(len, ((int64_t)T + 127) / 128, (int64_t)B * Hkv, 256 * (D == 64 ? 3 : 2), 16, pays);
 }
 
 template <int D>
@@ -530,15 +478,15 @@ hipError_t launch_bwd_dkdv(const BwdArgs& a, hipStream_t stream) {
   // four of them behind two tiles in flight; D = 128: four slots of 16 KB
   // (two per CU), three tiles in flight from the start.
   constexpr int NBUF = D == 64 ? 6 : 4, PRE = D == 64 ? 2 : 3;
-  if (a.split.n == 0) {
+  if (a.kchunks.n == 0) {
     hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, NBUF, PRE, false>), dim3((unsigned)(nkt * units)), dim3(kThreads), 0, stream, a);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, NBUF, PRE, true>), dim3((unsigned)(a.split.base[a.split.n] * units)),
+  hipLaunchKernelGGL((attn_bwd_dkdv_kernel<D, NBUF, PRE, true>), dim3((unsigned)(a.kchunks.base[a.kchunks.n] * units)),
                      dim3(kThreads), 0, stream, a);
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  const int64_t split_tiles = a.split.base[2] - a.split.base[1];
+  const int64_t split_tiles = a.kchunks.base[2] - a.kchunks.base[1];
   hipLaunchKernelGGL((attn_bwd_dkdv_merge_kernel<D>), dim3((unsigned)(split_tiles * units * 8)), dim3(kThreads), 0, stream, a);
   return hipGetLastError();
 }

@@ -26,6 +26,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace hlm {
 
 typedef __bf16 bf16;
@@ -65,17 +67,49 @@ struct FwdArgs {
   int nsplit;
 };
 
-// Split dK/dV (attn_bwd_dkdv.hip): the query tiles that a key tile meets are
-// cut into chunks of `len`, one workgroup each.  Chunk c exists for the key
-// tiles 0 .. base[c + 1] - base[c] - 1 (the count of query tiles never grows
-// with the key tile), and its partial sums are block base[c] + key tile of
-// `part`.  n = 0: not split.
-constexpr int kMaxDkdvChunks = 16;
-struct DkdvSplit {
+// A backward kernel's long tiles cut into chunks: a key tile's query tiles
+// (dK/dV) or a query tile's key tiles (dQ), `len` of them to a workgroup.  Rank
+// r is the key tile, or the query tile counted from the last one, so that the
+// count of tiles to visit does not grow with it (a ragged last query tile
+// aside).  Chunk c exists for ranks 0 .. base[c + 1] - base[c] - 1, and its
+// fp32 partial sums are block base[c] + rank of `part`.  n = 0: not cut.
+constexpr int kMaxChunks = 16;
+struct ChunkPlan {
   float* part;
   int len, n;
-  int base[kMaxDkdvChunks + 1];
+  int base[kMaxChunks + 1];
 };
+
+// The chunks of `ranks` tiles per unit with len(rank) steps each: the shortest
+// that fill the chip's workgroup slots once (at least min_len steps), if
+// pays(chunk length, chunks, longest tile) says that they beat whole tiles.
+template <class Len, class Pays>
+inline ChunkPlan plan_chunks(Len len, int64_t ranks, int64_t units, int slots, int64_t min_len, Pays pays) {
+  ChunkPlan s{};
+  if (units * ranks >= slots) return s;
+  int64_t total = 0, longest = 0;
+  for (int r = 0; r < ranks; ++r) {
+    total += len(r);
+    longest = std::max<int64_t>(longest, len(r));
+  }
+  int64_t c = std::max({(total * units + slots - 1) / slots, (longest + kMaxChunks - 1) / kMaxChunks, min_len});
+  int64_t blocks = 0;
+  for (; c < longest; c += std::max<int64_t>(c / 32, 1)) {
+    blocks = 0;
+    for (int r = 0; r < ranks; ++r) blocks += (len(r) + c - 1) / c;
+    blocks *= units;
+    if (blocks <= slots) break;
+  }
+  if (c >= longest || !pays(c, blocks, longest)) return s;
+  s.len = (int)c;
+  for (; s.n * c < longest; ++s.n) {
+    int has = 0;  // ranks up to the last one with a chunk s.n
+    for (int r = 0; r < ranks; ++r)
+      if (len(r) > s.n * c) has = r + 1;
+    s.base[s.n + 1] = s.base[s.n] + has;
+  }
+  return s;
+}
 
 struct BwdArgs {
   const bf16* q;
@@ -92,7 +126,7 @@ struct BwdArgs {
   int B, T, H, Hkv, W;
   float scale;       // softmax scale
   float scale_log2;  // scale * log2(e)
-  DkdvSplit split;
+  ChunkPlan qchunks, kchunks;  // of dQ and of dK/dV
 };
 
 // Arguments of the fused q/k RMSNorm + partial rotary kernels (qk_norm_rope.hip).
@@ -392,6 +426,42 @@ __device__ __forceinline__ bf16x8 lds_read_b128(unsigned addr) {
 __device__ __forceinline__ void lds_write_b64(unsigned addr, bf16x4 v) {
   typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
   *(lds_bf16x4*)(uintptr_t)addr = v;
+}
+
+// Adds n chunks' partial sums of 32 rows x D in their order, times f, and
+// stores the rows row0 .. that lie below T as bf16.  For a workgroup of 256:
+// thread (lane, wave) adds the f32x4 pieces wave, wave + 4, ... (accumulator
+// order, [db][i][lane]) from block(c), and the rows leave through the 64 D
+// bytes of LDS at `rows`.  Bound by reading the sums once, fully coalesced.
+template <int D, class Block>
+__device__ __forceinline__ void sum_chunk_rows(int n, Block block, float f, bf16* dst, int64_t stride, int row0, int T,
+                                               unsigned rows) {
+  using L = CS<D>;
+  constexpr int PPT = D / 32;  // f32x4 per thread and chunk
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  f32x4 acc[PPT];
+#pragma unroll
+  for (int p = 0; p < PPT; ++p) acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < n; ++c) {
+    const f32x4* s = block(c) + tid;
+#pragma unroll
+    for (int p = 0; p < PPT; ++p) acc[p] += s[p * 256];
+  }
+#pragma unroll
+  for (int p = 0; p < PPT; ++p) {
+    bf16x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (bf16)(acc[p][j] * f);
+    lds_write_b64(rows + L::byte(lane & 31, wave + 4 * p) + 8 * (lane >> 5), v);  // piece 4 db + i
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < (32 * L::U + 255) / 256; ++k) {
+    const int row = (tid + 256 * k) / L::U, u = tid % L::U;
+    if (row0 + row < T)
+      __builtin_nontemporal_store(lds_read_b128(rows + L::byte(row, u)),
+                                  reinterpret_cast<bf16x8*>(dst + (int64_t)(row0 + row) * stride + 8 * u));
+  }
 }
 
 }  // namespace hlm

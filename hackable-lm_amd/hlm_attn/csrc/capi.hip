@@ -1,5 +1,6 @@
 // extern "C" entry points of libhlm_attn.so (declared in include/hlm_attn.h):
 // argument validation, mask normalisation and kernel dispatch by head dim.
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -16,7 +17,8 @@ template <int D>
 int fwd_split_count(int B, int T, int H, int W);
 template <int D>
 hipError_t launch_bwd(const BwdArgs& a, hipStream_t stream, int phases);
-DkdvSplit dkdv_split_plan(int B, int T, int H, int Hkv, int D, int W);
+ChunkPlan dq_chunk_plan(int B, int T, int H, int D, int W);
+ChunkPlan dkdv_chunk_plan(int B, int T, int H, int Hkv, int D, int W);
 int fused_partial_slots(int T, int W);
 hipError_t launch_bwd_fused(const BwdArgs& a, bf16* part, int R, hipStream_t stream);
 template <int D>
@@ -184,14 +186,16 @@ int check_bwd(const void* q, const void* k, const void* v, const void* o, const 
 
 // phases: kBwdDq / kBwdDkDv / kBwdAll for the two-kernel backward, or
 // kBwdFused (with `part`, `part_bytes`) for the single-pass one; kBwdAll |
-// kBwdSplit (with `part`, `part_bytes`) cuts long dK/dV tiles into chunks
-// where dkdv_split_plan says so.
+// kBwdSplit (with `part`, `part_bytes`) cuts long dQ and dK/dV tiles into
+// chunks where their plans say so.
 constexpr int kBwdFused = 4;
 constexpr int kBwdSplit = 8;
 
-// Bytes of a split's partial sums: one fp32 dK and dV tile of 128 keys per chunk.
-int64_t split_bytes(const hlm::DkdvSplit& p, int B, int Hkv, int D) {
-  return (int64_t)p.base[p.n] * B * Hkv * 128 * D * 8;
+// Bytes of the chunks' partial sums: an fp32 dQ tile of 128 queries, or dK and
+// dV tiles of 128 keys, per chunk.  dQ's are summed before dK/dV's are written,
+// so the two share the workspace.
+int64_t chunk_bytes(const hlm::ChunkPlan& q, const hlm::ChunkPlan& k, int B, int H, int Hkv, int D) {
+  return std::max((int64_t)q.base[q.n] * B * H * 128 * D * 4, (int64_t)k.base[k.n] * B * Hkv * 128 * D * 8);
 }
 
 int run_bwd(int phases, const void* q, const void* k, const void* v, const void* o, const void* dout,
@@ -205,16 +209,17 @@ int run_bwd(int phases, const void* q, const void* k, const void* v, const void*
                      do_strides, dq_strides, dk_strides, dv_strides, scale);
   if (rc) return rc;
   int R = 0;
-  hlm::DkdvSplit split{};
+  hlm::ChunkPlan qchunks{}, kchunks{};
   if ((phases & kBwdSplit) && B > 0 && T > 0) {
-    split = hlm::dkdv_split_plan(B, T, H, Hkv, D, effective_window(window, T));
-    const int64_t need = split_bytes(split, B, Hkv, D);
+    qchunks = hlm::dq_chunk_plan(B, T, H, D, effective_window(window, T));
+    kchunks = hlm::dkdv_chunk_plan(B, T, H, Hkv, D, effective_window(window, T));
+    const int64_t need = chunk_bytes(qchunks, kchunks, B, H, Hkv, D);
     if (need > 0 && (part == nullptr || !aligned16(part)))
       return fail(HLM_ATTN_EINVAL, "partial workspace is null or not 16-byte aligned");
     if (part_bytes < need)
       return fail(HLM_ATTN_EINVAL, "partial workspace holds %lld bytes, %lld needed", (long long)part_bytes,
                   (long long)need);
-    split.part = static_cast<float*>(part);
+    qchunks.part = kchunks.part = static_cast<float*>(part);
   }
   if (phases == kBwdFused) {
     if (D != 64) return fail(HLM_ATTN_EUNSUPPORTED, "the single-pass backward takes head_dim 64 only (got %d)", D);
@@ -254,7 +259,8 @@ int run_bwd(int phases, const void* q, const void* k, const void* v, const void*
   a.W = effective_window(window, T);
   a.scale = scale;
   a.scale_log2 = scale * hlm::kLog2e;
-  a.split = split;
+  a.qchunks = qchunks;
+  a.kchunks = kchunks;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const hipError_t err = phases == kBwdFused ? hlm::launch_bwd_fused(a, static_cast<hlm::bf16*>(part), R, s)
                          : D == 64           ? hlm::launch_bwd<64>(a, s, phases)
@@ -368,7 +374,8 @@ int64_t hlm_attn_bwd_split_workspace_bytes(int B, int T, int H, int Hkv, int D, 
   g_last_error[0] = '\0';
   if (const int rc = check_dims(B, T, H, Hkv, D, 1.f)) return rc;
   if (B == 0 || T == 0) return 0;
-  return split_bytes(hlm::dkdv_split_plan(B, T, H, Hkv, D, effective_window(window, T)), B, Hkv, D);
+  const int W = effective_window(window, T);
+  return chunk_bytes(hlm::dq_chunk_plan(B, T, H, D, W), hlm::dkdv_chunk_plan(B, T, H, Hkv, D, W), B, H, Hkv, D);
 }
 
 int hlm_attn_bwd_split(const void* q, const void* k, const void* v, const void* o, const void* dout,

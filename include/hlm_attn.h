@@ -144,16 +144,17 @@ int hlm_attn_bwd_dkdv(const void* q, const void* k, const void* v, const void* o
                       int window, float scale, void* stream);
 
 /*
- * hlm_attn_bwd for small grids with long rows (few (batch, kv head) units,
- * long sequences, several query heads per kv head): a key tile's query tiles
- * are cut into chunks, one workgroup each, that write fp32 partial sums of
- * dk and dv to partial_ws, and a third kernel adds them in a fixed order
- * (deterministic).  partial_ws (16-byte aligned, no initialisation needed)
- * holds hlm_attn_bwd_split_workspace_bytes(B, T, H, Hkv, D, window) bytes,
- * passed as partial_ws_bytes; where that is 0 the call is hlm_attn_bwd (and
- * partial_ws may be null).  dq is hlm_attn_bwd's; dk and dv agree with it to
- * the order of the fp32 sums.  No counterpart in the reference:
- * FlashAttention-2's backward is one call.
+ * hlm_attn_bwd for small grids with long rows (few (batch, head) units, long
+ * sequences, several query heads per kv head): a query tile's key tiles, a key
+ * tile's query tiles, or both, are cut into chunks, one workgroup each, that
+ * write fp32 partial sums of dq, or of dk and dv, to partial_ws, and a merge
+ * kernel adds them in a fixed order (deterministic).  partial_ws (16-byte
+ * aligned, no initialisation needed) holds
+ * hlm_attn_bwd_split_workspace_bytes(B, T, H, Hkv, D, window) bytes, passed as
+ * partial_ws_bytes; where that is 0 the call is hlm_attn_bwd (and partial_ws
+ * may be null).  The gradients agree with hlm_attn_bwd's to the order of the
+ * fp32 sums.  No counterpart in the reference: FlashAttention-2's backward is
+ * one call.
  */
 int hlm_attn_bwd_split(const void* q, const void* k, const void* v, const void* o, const void* dout,
                        const float* lse, void* dq, void* dk, void* dv, float* delta_ws,
@@ -164,7 +165,7 @@ int hlm_attn_bwd_split(const void* q, const void* k, const void* v, const void* 
                        const int64_t* dk_strides, const int64_t* dv_strides,
                        int window, float scale, void* stream);
 /* Bytes of hlm_attn_bwd_split's partial workspace; 0 where splitting does not
- * pay (the key tiles fill the chip, or are short).  Negative: an HLM_ATTN_E*
+ * pay (the tiles fill the chip, or are short).  Negative: an HLM_ATTN_E*
  * code.  Pure function of the shape; touches no device. */
 int64_t hlm_attn_bwd_split_workspace_bytes(int B, int T, int H, int Hkv, int D, int window);
 

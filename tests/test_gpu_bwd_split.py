@@ -1,12 +1,13 @@
-"""The backward with long dK/dV tiles cut into chunks (hlm_attn_bwd_split): its
-argument checks and the shapes it applies to (CPU), and its results against
-hlm_attn_bwd and the fp32 oracle (GPU).
+"""The backward with long dQ and dK/dV tiles cut into chunks
+(hlm_attn_bwd_split): its argument checks and the shapes it applies to (CPU),
+and its results against hlm_attn_bwd and the fp32 oracle (GPU).
 
-dq comes from the same kernel and must be bit-identical.  dk and dv are the
-same fp32 products summed in another order and rounded to bf16 once, so two
-results differ by at most one bf16 step of the value (2^-7 relative) plus the
-fp32 sums' own reordering error, which is far below 1e-5 of the largest
-gradient.  Every call starts from a NaN-filled workspace.
+The gradients are the same fp32 products summed in another order and rounded
+to bf16 once, so two results differ by at most one bf16 step of the value
+(2^-7 relative) plus the fp32 sums' own reordering error, which is far below
+1e-5 of the largest gradient.  Where only one of dQ and dK/dV is cut, the
+other one's kernel is the same and its result bit-identical.  Every call
+starts from a NaN-filled workspace.
 """
 from __future__ import annotations
 
@@ -21,7 +22,7 @@ from oracle import attention as oracle
 from test_gpu_parity import assert_grad, make_inputs
 
 CASES = [
-    # B, T, H, Hkv, D, window
+    # B, T, H, Hkv, D, window: dK/dV cut, dQ as the sizes have it
     (1, 1, 64, 1, 64, None),      # one token, one key tile, 64 query heads: chunks of whole heads
     (1, 129, 32, 1, 128, None),   # a second key tile of one row
     (1, 300, 40, 2, 64, 40),      # short window, many heads: chunks end inside a head
@@ -31,18 +32,28 @@ CASES = [
     (2, 1777, 12, 4, 128, None),
     (1, 2048, 6, 6, 64, None),    # no grouping
 ]
+DQ_CASES = [
+    # dQ cut
+    (1, 1000, 4, 4, 128, None),   # ragged, two chunks
+    (1, 2048, 1, 1, 64, None),    # chunks of the shortest length
+    (2, 2049, 2, 2, 64, None),    # a last query tile of one row
+    (1, 2945, 2, 1, 64, 1944),    # windowed, and the ragged last query tile lacks the last chunk
+    (1, 3201, 2, 2, 128, 2000),
+    (1, 8192, 1, 1, 64, None),    # 16 chunks, the largest number
+]
 
 
 def _bytes(B, T, H, Hkv, D, window):
     return _lib.load().hlm_attn_bwd_split_workspace_bytes(B, T, H, Hkv, D, window or 0)
 
 
-@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("case", CASES + DQ_CASES)
 def test_split_applies_to_the_cases_below(case):
     B, T, H, Hkv, D, _ = case
     tiles, n = (T + 127) // 128, _bytes(*case)
-    block = B * Hkv * 128 * D * 8  # one chunk of every (batch, kv head): fp32 dK and dV of 128 keys
-    assert n % block == 0 and 2 * block <= n <= 16 * tiles * block
+    # One chunk of every (batch, kv head), fp32 dK and dV of 128 keys, or of every (batch, head), fp32 dQ.
+    kv_block, q_block = B * Hkv * 128 * D * 8, B * H * 128 * D * 4
+    assert any(n % b == 0 and 2 * b <= n <= 16 * tiles * b for b in (kv_block, q_block))
     assert n // (128 * D * 8) <= 256 * (3 if D == 64 else 2), "at most one filling of the chip"
 
 
@@ -79,7 +90,7 @@ def test_split_backward_checks_its_workspace():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("case", CASES + DQ_CASES)
 def test_split_backward_matches_the_unsplit_one_and_the_oracle(case):
     from hlm_attn import ops
 
@@ -111,9 +122,10 @@ def test_split_backward_matches_the_unsplit_one_and_the_oracle(case):
         torch.cuda.synchronize()
         got.append((dq, dk, dv))
     one, two, again = got
-    assert torch.equal(one[0], two[0])
+    # By the sizes, the first cases cut dK/dV only and the others dQ or both.
+    assert torch.equal(one[0], two[0]) == (case in CASES[:6])
     assert all(torch.equal(a, b) for a, b in zip(two, again)), "not deterministic"
-    for name, a, b in (("dk", one[1], two[1]), ("dv", one[2], two[2])):
+    for name, a, b in zip(("dq", "dk", "dv"), one, two):
         a, b = a.float(), b.float()
         assert bool(((a - b).abs() <= 2.0**-7 * a.abs() + 1e-5 * a.abs().max()).all()), name
     via_op = ops.hip_attn_bwd(dod, qd, kd, vd, o, lse, w, scale)
