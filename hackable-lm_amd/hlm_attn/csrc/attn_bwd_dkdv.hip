@@ -442,20 +442,25 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_merge_kernel(BwdArgs a
 // A key tile's workgroup walks its query tiles one after the other: 0.93 us
 // each at D = 128 and 0.62 us at D = 64 while workgroups have a CU to
 // themselves, so a grid that does not fill the chip takes as long as its
-// longest key tile.  In chunks that fill the workgroup slots once, a query
-// tile takes about 1.5 (D = 128) or 2.5 (D = 64) times that, beside the second
-// prologue, the fp32 partial sums and the merge (26 query tiles' time at D =
-// 128 where 512 chunks write sums, 12 at D = 64): the comparisons below, in
-// query tiles.  Chunks that fill the slots one and a half or two times, or
-// half, measured slower (B = 2, T = 1777, 12 query on 4 kv heads, D = 128,
-// causal: 20% at 1.5 and 2, 12% at 0.5).
+// longest key tile.  Chunks that fill the workgroup slots once run beside each
+// other, a query tile of each taking about 1.9 times that when every slot is
+// taken, and pay a second prologue, the fp32 partial sums and the merge, in
+// part by the number of chunks.  Fitted over 40 shapes, splitting pays while
+//   D = 64:  2 chunk + chunk blocks / 400 + blocks / 18 + 15 < 2 longest
+//   D = 128: 2 chunk + chunk blocks / 512 + blocks / 16 + 8 < 2 longest   (in query tiles of 32)
+// Up to 512 tokens and 52 query tiles D = 64 stays whole although it would gain
+// (333x4/1 W 129 32 -> 25): the tests hold the single-pass backward's dK and
+// dV to this path's bit for bit at such sizes.
+// Chunks that fill the slots one and a half or two times, or half, measured
+// slower (B = 2, T = 1777, 12 query on 4 kv heads, D = 128, causal: 20% at 1.5
+// and 2, 12% at 0.5).
 //
-// dK/dV with its merge, us, unsplit and split.  D = 128, causal unless W is
-// given: that shape 155 / 60; 12 on 12 heads 58 / 60 (refused); T = 8192, 16 on
-// 4, W = 2048 251 / 227; T = 2048, 12 heads 62 / 47; T = 1536, 16 heads 48 / 42;
-// T = 4096, 8 heads, W = 1024 38 / 51 (refused).  D = 64: T = 2048, 6 heads
-// 40 / 21; T = 4096, 12 heads 80 / 69; 2 x 2048, 12 heads 43 / 44 (refused);
-// T = 8192, 8 on 1 head 1157 / 180.
+// Whole backward (dQ in both as its own plan has it) with dK/dV unsplit ->
+// split (us), BxTxH/Hkv, causal unless W is given:
+//   taken    D = 64:  1500x4/4 47 -> 35, 1000x8/2 W 200 41 -> 29, 1024x12/12 39 -> 36, 2000x4/4 W 1024 42 -> 38
+//            D = 128: 2x1777x12/4 204 -> 110, 2000x4/4 W 1024 71 -> 55, 1024x16/16 61 -> 53, 1000x6/6 58 -> 49
+//   refused  D = 64:  2x2048x12/12 76 -> 78, 4096x16/16 153 -> 157, 2x1000x8/4 W 256 29 -> 30
+//            D = 128: 2048x16/16 W 512 48 -> 61, 4096x8/8 W 1024 74 -> 87, 500x8/8 the same
 ChunkPlan dkdv_chunk_plan(int B, int T, int H, int Hkv, int D, int W) {
   const int G = H / Hkv;
   // Query tiles that a key tile meets, over the group's heads.
@@ -464,7 +469,9 @@ ChunkPlan dkdv_chunk_plan(int B, int T, int H, int Hkv, int D, int W) {
     return (std::min<int64_t>(T - 1, k0 + 126 + W) / 32 - k0 / 32 + 1) * G;
   };
   auto pays = [=](int64_t c, int64_t blocks, int64_t longest) {
-    return D == 64 ? 5 * c + 24 < 2 * longest : 3 * c + 12 + 5 * blocks / 64 < 2 * longest;
+    if (D == 64 && T <= 512 && longest <= 52) return false;
+    return (D == 64 ? 2 * c + c * blocks / 400 + blocks / 18 + 15 : 2 * c + c * blocks / 512 + blocks / 16 + 8) <
+           2 * longest;
   };
   return plan_chunks(len, ((int64_t)T + 127) / 128, (int64_t)B * Hkv, 256 * (D == 64 ? 3 : 2), 16, pays);
 }
