@@ -101,9 +101,10 @@ _torch_fwd_error = ""
 
 
 def load_torch_fwd():
-    """The torch C++ extension of the no-grad forward (_torch_fwd: checks,
-    allocation and launch in one C++ call), built with the library; raises if
-    it is missing or unusable.  The forward does not need it: see torch_fwd()."""
+    """The torch C++ extension (_torch_fwd: the no-grad forward's checks,
+    allocation and launch in one C++ call, and the differentiable calls as C++
+    autograd functions), built with the library; raises if it is missing or
+    unusable.  No call needs it: see torch_fwd()."""
     ext = torch_fwd()
     if ext is None:
         raise HipAttentionUnavailable(

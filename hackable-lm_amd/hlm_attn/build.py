@@ -1,6 +1,6 @@
 """Builds libhlm_attn.so (the HIP kernels + C ABI) for gfx950 with hipcc, the
 CPython binding of its forward entry points (_pycall, host code, g++) and the
-torch C++ extension of the no-grad forward (_torch_fwd, host code).
+torch C++ extension of plain eager calls (_torch_fwd, host code).
 
 Both are built in-tree next to this file, so they travel with the source tree
 to the GPU host.  Usage:  python -m hlm_attn.build  (or build()).
