@@ -421,26 +421,38 @@ hipError_t launch_fwd(const FwdArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Splits for a small forward grid.  A workgroup alone on a CU runs a key
-// tile in about 1 us (latency-bound), three sharing a CU about 2.1 us each,
-// and the merge pass costs 4-10 us (measured on the MI355X at B = 1, H = 12,
-// D = 64).  So splitting pays only when the longest row is long: 1 (no
-// split) when the tiles already occupy half of the workgroup slots or the
-// longest row has fewer than 24 key tiles; otherwise one split per 12 key
-// tiles of the longest row, at most enough to fill the slots and at most
-// kMaxSplit.  (B = 1, T = 2048, causal: 33.7 us unsplit, 28 us in 2 splits;
-// with a 512-key window, or at T = 1024, splitting is slower.)
+// Splits for a small forward grid: the n that share a query tile's key range,
+// or 1.  A workgroup alone on a CU runs a key tile of 64 in 0.8 us (D = 128:
+// 1.2), latency-bound, so an idle chip takes as long as its longest row; n
+// runs divide that, share their CUs, and pay partial results and a merge pass
+// that grow with n.  One run per 12 key tiles, at most enough to fill the
+// slots; few units take up to four runs of at least 5.  In key tiles, L the
+// longest row's, splitting pays while
+//   2 (L - all rows' tiles / 320) > 26 + n workgroups / 40
+// (fitted over 55 shapes, B = 1 unless given, heads on as many kv heads):
+//            T x heads, causal or W     unsplit, split in n (us)
+//   D = 64:  2047x12 29.6, 2: 26.1;  4000x12 54.3, 2: 47.8;  1024x4 16.2, 3: 13.9;
+//            1500x4 22.9, 4: 16.2;  2000x4 W 1024 18.6, 3: 16.3
+//   D = 128: 1500x6 31.0, 4: 22.9;  4000x12 79.7, 2: 69.9;  1024x4 21.9, 3: 17.2
+//   refused  D = 64: 4000x16 55.2, 2: 56.6;  6000x8 W 3000 45.0, 3: 50.6;
+//            2047x12 W 1024 18.7, 2: 22.7;  D = 128: 2 x 1777x12 38.3, 2: 41.5
 template <int D>
 int fwd_split_count(int B, int T, int H, int W) {
-  constexpr int BM = 128, BN = 64, kMaxSplit = 16, kMinTiles = 24, kTilesPerSplit = 12;
+  constexpr int BM = 128, BN = 64, kMaxSplit = 16;
   const int slots = 256 * (D == 64 ? 3 : 2);  // resident workgroups on the MI355X
-  const int64_t units = (int64_t)((T + BM - 1) / BM) * B * H;
-  if (units == 0 || 2 * units >= slots) return 1;
-  const int longest = (min(T, W + BM - 1) + BN - 1) / BN + 1;  // key tiles of the longest row
-  if (longest < kMinTiles) return 1;
-  const int fill = (int)((slots + units - 1) / units);
-  const int n = min(min(longest / kTilesPerSplit, fill), kMaxSplit);
-  return n >= 2 ? n : 1;
+  const int64_t units = ((int64_t)T + BM - 1) / BM * B * H;
+  if (units == 0 || units >= slots) return 1;
+  int64_t longest = 0, total = 0;  // key tiles of the longest row, of all
+  for (int64_t q0 = 0; q0 < T; q0 += BM) {
+    const int64_t len = (min((int64_t)T, q0 + BM) - 1) / BN - max((int64_t)0, q0 - W + 1) / BN + 1;
+    longest = max(longest, len);
+    total += len * B * H;
+  }
+  if (longest < 16) return 1;
+  const int64_t fill = (slots + units - 1) / units;
+  const int64_t runs = max(longest / 12, units < 4 * longest ? min(longest / 5, (int64_t)4) : (int64_t)1);
+  const int64_t n = min(min(runs, fill), (int64_t)kMaxSplit);
+  return n >= 2 && 2 * (longest - total / 320) > 26 + n * units / 40 ? (int)n : 1;
 }
 
 template int fwd_split_count<64>(int, int, int, int);

@@ -95,11 +95,11 @@ int hlm_attn_fwd_split(const void* q, const void* k, const void* v, void* o, flo
 
 /*
  * The nsplit this library recommends for hlm_attn_fwd_split on an MI355X:
- * 1 (use hlm_attn_fwd) unless the query tiles fill less than half of the
- * chip's workgroup slots and the longest row spans at least 24 key tiles of
- * 64 (shorter rows run faster unsplit than split and merged); then one split
- * per 12 key tiles of the longest row.  Pure function of the shape; touches
- * no device.
+ * 1 (use hlm_attn_fwd) where the query tiles fill the chip's workgroup slots,
+ * the longest row spans fewer than 16 key tiles of 64, or the longest row's
+ * walk is not what takes the time; else one split per 12 key tiles of the
+ * longest row, or up to four of five key tiles where there are few query
+ * tiles.  Pure function of the shape; touches no device.
  */
 int hlm_attn_fwd_split_count(int B, int T, int H, int D, int window);
 
