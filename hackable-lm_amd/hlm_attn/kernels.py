@@ -286,6 +286,11 @@ class _LMHeadLoss(torch.autograd.Function):
         padded[:, vocab:] = 0  # hip_ce_dhidden's contract; nothing writes there
         work = padded[:, :vocab]
         w_t = weight.t()
+        # Plain eager programs call the launches behind the two custom ops: the
+        # dispatcher's host time is what a loss of a few hundred tokens waits for.
+        plain = ops.eager_ext(hidden, weight, targets) is not None
+        ce_rows = ops.linear_ce_impl if plain else ops.hip_linear_ce_into
+        ce_dhidden = ops.ce_dhidden_impl if plain else ops.hip_ce_dhidden
         for r0 in range(0, n, rows):
             r1 = min(r0 + rows, n)
             h = hidden[r0:r1]
@@ -294,9 +299,9 @@ class _LMHeadLoss(torch.autograd.Function):
                 torch.mm(h, w_t, out=g)
             else:
                 torch.addmm(bias, h, w_t, out=g)
-            ops.hip_linear_ce_into(g, targets[r0:r1], n, losses[r0:r1])
+            ce_rows(g, targets[r0:r1], n, losses[r0:r1])
             if want_h:
-                ops.hip_ce_dhidden(padded[: r1 - r0], weight, vocab, d_hidden[r0:r1])
+                ce_dhidden(padded[: r1 - r0], weight, vocab, d_hidden[r0:r1])
             if want_w and r0 == 0:
                 torch.mm(g.t(), h, out=d_weight)
             elif want_w:

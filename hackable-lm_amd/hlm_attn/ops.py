@@ -503,11 +503,8 @@ def _ce_dhidden_ready(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, ou
     return _lib.load().hlm_ce_dhidden_pays(work.shape[0], weight.shape[1], n_vocab) == 1
 
 
-@torch.library.custom_op("hackable_lm::hip_ce_dhidden", mutates_args=("out",))
-def hip_ce_dhidden(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> None:
-    """out = work[:, :n_vocab] @ weight, where work's columns from n_vocab to the
-    next multiple of 64 hold zeros.  The choice between hlm_ce_dhidden and the
-    library's product is made here, so that a trace holds one op."""
+def ce_dhidden_impl(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> None:
+    """The product behind hackable_lm::hip_ce_dhidden."""
     rows, n = work.shape[0], weight.shape[1]
     if weight.shape[0] != n_vocab or out.shape != (rows, n) or work.shape[1] < -(-n_vocab // 64) * 64:
         raise RuntimeError(f"work {tuple(work.shape)}, weight {tuple(weight.shape)} and out {tuple(out.shape)} do not match")
@@ -523,6 +520,14 @@ def hip_ce_dhidden(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: 
             rows, n, n_vocab, None if ws is None else ws.data_ptr(), nbytes, _stream_handle(work.device),
         )
     _lib.check(rc, lib)
+
+
+@torch.library.custom_op("hackable_lm::hip_ce_dhidden", mutates_args=("out",))
+def hip_ce_dhidden(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> None:
+    """out = work[:, :n_vocab] @ weight, where work's columns from n_vocab to the
+    next multiple of 64 hold zeros.  The choice between hlm_ce_dhidden and the
+    library's product is made here, so that a trace holds one op."""
+    ce_dhidden_impl(work, weight, n_vocab, out)
 
 
 @hip_ce_dhidden.register_fake
