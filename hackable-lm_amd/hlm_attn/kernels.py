@@ -269,8 +269,8 @@ class _LMHeadLoss(torch.autograd.Function):
         n, d = hidden.shape
         vocab = weight.shape[0]
         rows = linear_ce_chunk_size(n, d, vocab, requested_chunk_size)
-        want_h, want_w = hidden.requires_grad, weight.requires_grad
-        want_b = bias is not None and bias.requires_grad
+        # (not from hidden and weight: a contiguous copy does not require grad here)
+        want_h, want_w, _, want_b, _ = ctx.needs_input_grad
         d_hidden = torch.empty_like(hidden) if want_h else None
         d_weight = torch.empty_like(weight) if want_w else None
         d_bias = torch.zeros_like(bias) if want_b else None
