@@ -249,67 +249,34 @@ class _LMHeadLoss(torch.autograd.Function):
 
     The rows are processed in chunks (`linear_ce_chunk_size`).  One logits
     workspace of chunk x V is allocated once and every chunk's GEMM writes
-    into it; the HIP row kernel (hackable_lm::hip_linear_ce_into) turns it in
-    place into the gradient of the mean loss and writes the rows' losses.
-    The three gradient products are formed in the forward, straight into
-    their destinations: dhidden rows by a GEMM whose output is the chunk's
-    slice of the dhidden buffer (hackable_lm::hip_ce_dhidden where it beats the
-    library's), dW written by the first chunk's GEMM and accumulated inside the
-    others' (addmm_, one rounding per chunk), db by an in-place add.  The backward only scales the
-    three by the incoming gradient.  The results match the reference's
-    chunked loop (kernels.py:878-942), which this replaces."""
+    into it; the HIP row kernel turns it in place into the gradient of the
+    mean loss and writes the rows' losses.  The three gradient products are
+    formed in the forward, straight into their destinations: dhidden rows by a
+    GEMM whose output is the chunk's slice of the dhidden buffer (the library's
+    or hlm_ce_dhidden, whichever is faster), dW written by the first chunk's
+    GEMM and accumulated inside the others' (addmm_, one rounding per chunk),
+    db by an in-place add.  The backward only scales the three by the incoming
+    gradient.  The results match the reference's chunked loop
+    (kernels.py:878-942), which this replaces.
+
+    Plain eager programs run the loop directly: the dispatcher's host time is
+    what a loss of a few hundred tokens waits for.  Others, torch.compile among
+    them, see it as one op (hackable_lm::hip_lm_head_loss)."""
 
     @staticmethod
     def forward(ctx, hidden, weight, targets, bias, requested_chunk_size):
         from . import ops
 
-        hidden = hidden.contiguous()
-        weight = weight.contiguous()
-        targets = targets.contiguous()
         n, d = hidden.shape
-        vocab = weight.shape[0]
-        rows = linear_ce_chunk_size(n, d, vocab, requested_chunk_size)
-        # (not from hidden and weight: a contiguous copy does not require grad here)
+        rows = linear_ce_chunk_size(n, d, weight.shape[0], requested_chunk_size)
+        # (not from contiguous copies of hidden and weight: they do not require grad here)
         want_h, want_w, _, want_b, _ = ctx.needs_input_grad
-        d_hidden = torch.empty_like(hidden) if want_h else None
-        d_weight = torch.empty_like(weight) if want_w else None
-        d_bias = torch.zeros_like(bias) if want_b else None
-        losses = torch.empty(n, dtype=torch.float32, device=hidden.device)
-        # Rows of the workspace start on 128-byte lines: with V = 50257 the three
-        # products of a 4096-row chunk take 1132 us instead of 1275.
-        # They are not a multiple of 4 KB apart, which would put a column of them
-        # on few memory channels (dhidden 217 instead of 176 us at V = 32768).
-        stride = -(-vocab // 64) * 64
-        if stride * hidden.element_size() % 4096 == 0:
-            stride += 64
-        padded = hidden.new_empty((rows, stride))
-        padded[:, vocab:] = 0  # hip_ce_dhidden's contract; nothing writes there
-        work = padded[:, :vocab]
-        w_t = weight.t()
-        # Plain eager programs call the launches behind the two custom ops: the
-        # dispatcher's host time is what a loss of a few hundred tokens waits for.
-        plain = ops.eager_ext(hidden, weight, targets) is not None
-        ce_rows = ops.linear_ce_impl if plain else ops.hip_linear_ce_into
-        ce_dhidden = ops.ce_dhidden_impl if plain else ops.hip_ce_dhidden
-        for r0 in range(0, n, rows):
-            r1 = min(r0 + rows, n)
-            h = hidden[r0:r1]
-            g = work[: r1 - r0]
-            if bias is None:
-                torch.mm(h, w_t, out=g)
-            else:
-                torch.addmm(bias, h, w_t, out=g)
-            ce_rows(g, targets[r0:r1], n, losses[r0:r1])
-            if want_h:
-                ce_dhidden(padded[: r1 - r0], weight, vocab, d_hidden[r0:r1])
-            if want_w and r0 == 0:
-                torch.mm(g.t(), h, out=d_weight)
-            elif want_w:
-                d_weight.addmm_(g.t(), h)
-            if want_b:
-                d_bias.add_(g.sum(dim=0).to(d_bias.dtype))
-        ctx.save_for_backward(d_hidden, d_weight, d_bias)
-        return losses.sum()
+        tensors = (hidden, weight, targets) if bias is None else (hidden, weight, targets, bias)
+        plain = ops.eager_ext(*tensors) is not None
+        run = ops.lm_head_loss_impl if plain else ops.hip_lm_head_loss
+        loss, *grads = run(hidden, weight, bias, targets, rows, want_h, want_w, want_b)
+        ctx.save_for_backward(*(t if want else None for t, want in zip(grads, (want_h, want_w, want_b))))
+        return loss
 
     @staticmethod
     def backward(ctx, grad_output):

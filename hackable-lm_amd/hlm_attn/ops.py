@@ -23,6 +23,7 @@ import os
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils.flop_counter import register_flop_formula
 
 from . import _lib
 
@@ -484,17 +485,6 @@ def _(logits, targets, n_tokens):
     return logits.new_empty((logits.shape[0],), dtype=torch.float32)
 
 
-@torch.library.custom_op("hackable_lm::hip_linear_ce_into", mutates_args=("logits", "loss"))
-def hip_linear_ce_into(logits: torch.Tensor, targets: torch.Tensor, n_tokens: int, loss: torch.Tensor) -> None:
-    """hip_linear_ce with the rows' losses written to `loss`."""
-    linear_ce_impl(logits, targets, n_tokens, loss)
-
-
-@hip_linear_ce_into.register_fake
-def _(logits, targets, n_tokens, loss):
-    return None
-
-
 def _ce_dhidden_ready(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> bool:
     """True where hlm_ce_dhidden takes these tensors and beats the library's product."""
     if not all(t.is_cuda and t.dtype is _BF16 and t.stride(1) == 1 and not (t.stride(0) & 7 or t.data_ptr() & 15)
@@ -525,14 +515,88 @@ def ce_dhidden_impl(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out:
 @torch.library.custom_op("hackable_lm::hip_ce_dhidden", mutates_args=("out",))
 def hip_ce_dhidden(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> None:
     """out = work[:, :n_vocab] @ weight, where work's columns from n_vocab to the
-    next multiple of 64 hold zeros.  The choice between hlm_ce_dhidden and the
-    library's product is made here, so that a trace holds one op."""
+    next multiple of 64 hold zeros: hlm_ce_dhidden, or the library's product."""
     ce_dhidden_impl(work, weight, n_vocab, out)
 
 
 @hip_ce_dhidden.register_fake
 def _(work, weight, n_vocab, out):
     return None
+
+
+def lm_head_loss_impl(
+    hidden: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, targets: torch.Tensor,
+    rows: int, want_h: bool, want_w: bool, want_b: bool,
+) -> tuple[torch.Tensor, torch.Tensor | None, torch.Tensor | None, torch.Tensor | None]:
+    """The chunk loop behind hackable_lm::hip_lm_head_loss: the mean loss and
+    its gradients of hidden, weight and bias (None where not wanted)."""
+    hidden = hidden.contiguous()
+    weight = weight.contiguous()
+    targets = targets.contiguous()
+    n, vocab = hidden.shape[0], weight.shape[0]
+    d_hidden = hidden.new_empty(hidden.shape) if want_h else None
+    d_weight = weight.new_empty(weight.shape) if want_w else None
+    d_bias = bias.new_zeros(bias.shape) if want_b else None
+    losses = torch.empty(n, dtype=torch.float32, device=hidden.device)
+    # Rows of the workspace start on 128-byte lines: with V = 50257 the three
+    # products of a 4096-row chunk take 1132 us instead of 1275.
+    # They are not a multiple of 4 KB apart, which would put a column of them
+    # on few memory channels (dhidden 217 instead of 176 us at V = 32768).
+    stride = -(-vocab // 64) * 64
+    if stride * hidden.element_size() % 4096 == 0:
+        stride += 64
+    padded = hidden.new_empty((rows, stride))
+    padded[:, vocab:] = 0  # ce_dhidden_impl's contract; nothing writes there
+    work = padded[:, :vocab]
+    w_t = weight.t()
+    for r0 in range(0, n, rows):
+        r1 = min(r0 + rows, n)
+        h = hidden[r0:r1]
+        g = work[: r1 - r0]
+        if bias is None:
+            torch.mm(h, w_t, out=g)
+        else:
+            torch.addmm(bias, h, w_t, out=g)
+        linear_ce_impl(g, targets[r0:r1], n, losses[r0:r1])
+        if d_hidden is not None:
+            ce_dhidden_impl(padded[: r1 - r0], weight, vocab, d_hidden[r0:r1])
+        if d_weight is not None:
+            if r0 == 0:
+                torch.mm(g.t(), h, out=d_weight)
+            else:
+                d_weight.addmm_(g.t(), h)
+        if d_bias is not None:
+            d_bias.add_(g.sum(dim=0).to(d_bias.dtype))
+    return losses.sum(), d_hidden, d_weight, d_bias
+
+
+@torch.library.custom_op("hackable_lm::hip_lm_head_loss", mutates_args=())
+def hip_lm_head_loss(
+    hidden: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, targets: torch.Tensor,
+    rows: int, want_h: bool, want_w: bool, want_b: bool,
+) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """The loss of all chunks of `rows` tokens as one op: a trace holds neither
+    the logits workspace, whose padded rows are no `out=` that torch.compile
+    takes, nor the launches.  Gradients that are not wanted come back empty."""
+    loss, *grads = lm_head_loss_impl(hidden, weight, bias, targets, rows, want_h, want_w, want_b)
+    return (loss, *(hidden.new_empty(0) if t is None else t for t in grads))
+
+
+@hip_lm_head_loss.register_fake
+def _(hidden, weight, bias, targets, rows, want_h, want_w, want_b):
+    none = hidden.new_empty
+    return (
+        hidden.new_empty((), dtype=torch.float32),
+        hidden.new_empty(hidden.shape) if want_h else none(0),
+        weight.new_empty(weight.shape) if want_w else none(0),
+        bias.new_empty(bias.shape) if want_b else none(0),
+    )
+
+
+@register_flop_formula(torch.ops.hackable_lm.hip_lm_head_loss)
+def _lm_head_loss_flops(hidden_shape, weight_shape, bias_shape, targets_shape, rows, want_h, want_w, want_b, **kwargs) -> int:
+    """The products inside the op, which torch's FLOP counter does not see."""
+    return 2 * hidden_shape[0] * weight_shape[0] * weight_shape[1] * (1 + want_h + want_w)
 
 
 # --- residual add + RMSNorm after the output / down projections -------------------

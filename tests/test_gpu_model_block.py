@@ -45,10 +45,10 @@ class Block(torch.nn.Module):
         return loss
 
 
-def _make(dev):
+def _make(dev, vocab):
     from hlm_attn import AttentionConfig
 
-    cfg = AttentionConfig(n_layer=2, n_head=4, n_kv_head=4, n_embd=256, head_dim=64, vocab_size=512,
+    cfg = AttentionConfig(n_layer=2, n_head=4, n_kv_head=4, n_embd=256, head_dim=64, vocab_size=vocab,
                           attention_window=64, loss_chunk_size=None)
     torch.manual_seed(0)
     block = Block(cfg, 0).to(dev)
@@ -57,7 +57,7 @@ def _make(dev):
     g = torch.Generator().manual_seed(1)
     x = torch.randn(2, 96, 256, generator=g).bfloat16()
     res = torch.randn(2, 96, 256, generator=g).bfloat16()
-    targets = torch.randint(0, 512, (2, 96), generator=g)
+    targets = torch.randint(0, vocab, (2, 96), generator=g)
     return cfg, block, x, res, targets
 
 
@@ -74,14 +74,16 @@ def _reference_loss(cfg, block, x, res, targets):
     q, k = qk_oracle.qk_norm_rope(q, k, cos.float(), sin.float(), cfg.norm_eps)
     y = attn_oracle.attention_core_torch(q, k, v, 64)
     out, normed = res_oracle.residual_rms_norm(rf, y.reshape(2, 96, 256) @ w_o.t(), cfg.norm_eps)
-    loss = F.cross_entropy((normed @ w_head.t()).reshape(-1, 512), targets.reshape(-1))
+    loss = F.cross_entropy((normed @ w_head.t()).reshape(-1, cfg.vocab_size), targets.reshape(-1))
     loss.backward()
     return loss.detach(), w_qkv.grad
 
 
-def test_block_matches_reference_formulas_and_compiles():
+@pytest.mark.parametrize("vocab", [512, 1000, 32768])
+def test_block_matches_reference_formulas_and_compiles(vocab):
     dev = _dev()
-    cfg, block, x, res, targets = _make(dev)
+    torch._dynamo.reset()
+    cfg, block, x, res, targets = _make(dev, vocab)
     ref_loss, ref_gw = _reference_loss(cfg, block, x, res, targets)
 
     results = []

@@ -1,11 +1,15 @@
 """The LM-head loss's chunk loop (kernels._LMHeadLoss) on the CPU: the library
 products run as on the GPU, the cross-entropy rows come from the oracle in
-place of their launch."""
+place of their launch.  And how torch.compile sees the loss: traced with fake
+ROCm tensors."""
 from __future__ import annotations
 
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils.flop_counter import FlopCounterMode
 
+import hlm_attn
 from hlm_attn import kernels, ops
 from oracle import linear_ce as oracle
 
@@ -66,3 +70,49 @@ def test_only_the_wanted_gradients_are_formed(cpu_rows, wanted):
     loss = kernels._LMHeadLoss.apply(ins[0], ins[1], torch.randint(0, 5, (20,)), ins[2], None)
     loss.backward()
     assert [t.grad is not None for t in ins] == [i in wanted for i in range(3)]
+
+
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("vocab", [512, 1000, 2048, 32768, 50257, 65536])
+def test_loss_traces_with_fullgraph_as_one_op(vocab, with_bias):
+    """The reference trains under torch.compile(fullgraph=True)
+    (kernels.py:126-137).  Vocabularies whose workspace rows are padded, for
+    their alignment or off a multiple of 4 KB, and ones whose rows are not."""
+    calls = []
+
+    def backend(gm, example_inputs):
+        calls.extend(str(n.target) for m in gm.modules() if isinstance(m, torch.fx.GraphModule)
+                     for n in m.graph.nodes if n.op == "call_function")
+        return gm.forward
+
+    def loss_of(h, w, b, t):
+        return hlm_attn.fused_linear_cross_entropy_with_weight(h, w, b, t, chunk_size=2048)
+
+    torch._dynamo.reset()
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        h, w, b = (torch.empty(s, dtype=torch.bfloat16, device="cuda", requires_grad=True)
+                   for s in ((2500, 64), (vocab, 64), (vocab,)))
+        targets = torch.empty(2500, dtype=torch.int64, device="cuda")
+        loss = torch.compile(loss_of, fullgraph=True, backend=backend)(h, w, b if with_bias else None, targets)
+    assert loss.shape == () and loss.dtype == torch.float32
+    assert [c for c in calls if "hackable_lm" in c] == ["hackable_lm.hip_lm_head_loss.default"], calls
+
+
+@pytest.mark.parametrize("wanted,products", [((), 1), ((0,), 2), ((0, 1, 2), 3)])
+def test_the_op_and_the_direct_loop_agree(cpu_rows, wanted, products):
+    """A dispatch mode sees the op, with the FLOPs of its products."""
+    g = torch.Generator().manual_seed(4)
+    ins = [torch.randn(s, generator=g) for s in ((2100, 8), (65, 8), (65,))]
+    for i in wanted:
+        ins[i].requires_grad_(True)
+    targets = torch.randint(0, 65, (2100,), generator=g)
+
+    def once():
+        loss = kernels._LMHeadLoss.apply(ins[0], ins[1], targets, ins[2], 2048)
+        return (loss.detach(), *(torch.autograd.grad(loss, [ins[i] for i in wanted]) if wanted else ()))
+
+    direct = once()
+    with FlopCounterMode(display=False) as flops:
+        op = once()
+    assert flops.get_total_flops() == products * 2 * 2100 * 65 * 8
+    assert all(torch.equal(a, b) for a, b in zip(direct, op))
