@@ -544,9 +544,12 @@ int hlm_ce_dhidden(const void* grad, int64_t grad_stride, const void* weight, in
   g_last_error[0] = '\0';
   if (const int rc = check_ce_dhidden(n_rows, n_hidden, n_vocab)) return rc;
   const int64_t padded = ((int64_t)n_vocab + 63) / 64 * 64;
-  if (grad_stride < padded || grad_stride % 8 != 0 || grad_stride > (1 << 21))
-    return fail(HLM_ATTN_EINVAL, "grad stride %lld must be a multiple of 8 in [%lld, 2^21]", (long long)grad_stride,
-                (long long)padded);
+  // The longest vocabulary's rows and 64 columns to keep them off a multiple
+  // of 4 KB (a tile's 256 rows stay below 2^31 bytes).
+  constexpr int64_t max_stride = (1 << 21) + 64;
+  if (grad_stride < padded || grad_stride % 8 != 0 || grad_stride > max_stride)
+    return fail(HLM_ATTN_EINVAL, "grad stride %lld must be a multiple of 8 in [%lld, %lld]", (long long)grad_stride,
+                (long long)padded, (long long)max_stride);
   if (weight_stride < n_hidden || weight_stride % 8 != 0 || weight_stride > (1 << 22))
     return fail(HLM_ATTN_EINVAL, "weight stride %lld must be a multiple of 8 in [%d, 2^22]", (long long)weight_stride, n_hidden);
   if (dhidden_stride < n_hidden || dhidden_stride % 8 != 0)

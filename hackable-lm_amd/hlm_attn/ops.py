@@ -487,9 +487,12 @@ def _(logits, targets, n_tokens):
 
 def _ce_dhidden_ready(work: torch.Tensor, weight: torch.Tensor, n_vocab: int, out: torch.Tensor) -> bool:
     """True where hlm_ce_dhidden takes these tensors and beats the library's product."""
-    if not all(t.is_cuda and t.dtype is _BF16 and t.stride(1) == 1 and not (t.stride(0) & 7 or t.data_ptr() & 15)
-               for t in (work, weight, out)):
-        return False
+    for t, longest in ((work, (1 << 21) + 64), (weight, 1 << 22), (out, 1 << 62)):
+        if not t.is_cuda or t.dtype is not _BF16 or t.data_ptr() & 15:
+            return False
+        row, col = t.stride()
+        if col != 1 or row & 7 or not t.shape[1] <= row <= longest:
+            return False
     return _lib.load().hlm_ce_dhidden_pays(work.shape[0], weight.shape[1], n_vocab) == 1
 
 

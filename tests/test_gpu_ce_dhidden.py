@@ -62,6 +62,35 @@ def test_arguments_are_checked_before_touching_the_device():
     assert call(M=0) == 0
 
 
+@pytest.mark.parametrize("vocab", [2097088, 2097089, 2097152, 2097153])
+def test_the_rule_and_the_stride_check_agree_at_the_longest_vocabularies(vocab):
+    """Where the rule says yes, the loss's workspace rows (a multiple of 64, and
+    64 more where that is a multiple of 4 KB) are taken."""
+    lib = _lib.load()
+    stride = -(-vocab // 64) * 64
+    stride += 64 * (stride * 2 % 4096 == 0)
+    p = ctypes.c_void_p(0x1000)
+    rc = lib.hlm_ce_dhidden(p, stride, p, 64, p, 64, 0, 64, vocab, p, 1 << 40, None)
+    assert (rc == 0) == (lib.hlm_ce_dhidden_pays(1, 64, vocab) == 1) == (vocab <= 1 << 21), lib.hlm_attn_last_error()
+
+
+def test_op_leaves_strides_that_the_kernel_refuses_to_the_library(monkeypatch):
+    """The row stride of a single row may be anything, also below its length."""
+    from hlm_attn import ops
+
+    class OnDevice(torch.Tensor):
+        is_cuda = True
+
+    def row(cols, stride):
+        return torch.zeros(64, dtype=torch.bfloat16).as_strided((1, cols), (stride, 1)).as_subclass(OnDevice)
+
+    monkeypatch.setattr(_lib.load(), "hlm_ce_dhidden_pays", lambda *a: 1)
+    assert ops._ce_dhidden_ready(row(64, 64), row(32, 32), 1, row(32, 32))
+    for strides in ((8, 32, 32), (64, 0, 32), (64, 8, 32), (64, 32, 24), (64, 1 << 23, 32), (1 << 22, 32, 32)):
+        work, weight, out = (row(c, s) for c, s in zip((64, 32, 32), strides))
+        assert not ops._ce_dhidden_ready(work, weight, 1, out), strides
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,hidden,vocab", CASES)
 def test_matches_the_product_of_the_same_operands(rows, hidden, vocab):
