@@ -244,16 +244,22 @@ int lm_head_dhidden_runs(int M, int N, int K) {
   return (steps + per - 1) / per;  // every run has work
 }
 
-// Whether the kernels above beat a product that does not split K: few tiles,
-// and the runs fill the CUs.  us, this / the library's: 4096 x 768 (48 tiles,
-// 240 workgroups) 176 / 322, 4096 x 320 145 / 258, 300 x 256 x 1000 15 / 20;
-// 4096 x 2048 (128 tiles, 256 workgroups) 420 / 428; 8192 x 768 (96 tiles, 192
-// workgroups) 374 / 352: refused, as are more tiles.
+// Whether the kernels above beat a product that does not split K: few tiles
+// whose runs can fill the CUs, and a K that is long against what a split pays
+// before its first and after its last product (12 us with 100 columns, where
+// the library takes 5).  Kernel times in us, this / the library's (585 sizes,
+// rows x hidden x vocabulary):
+//   taken    4096 x 768 x 32768 194 / 319, x 6000 53 / 79; 272 x 256 x 4000 18 / 20;
+//            4096 x 512 x 4000 38 / 43; 3000 x 768 x 6000 64 / 63; 4096 x 2048 x 6000 101 / 106
+//   refused  by K: 272 x 256 x 900 25 / 9, x 3000 19 / 16; 4096 x 1024 x 2000 39 / 30, x 4000 52 / 51;
+//            3000 x 768 x 4000 51 / 41; 4096 x 2048 x 4000 78 / 73
+//            by the CUs: 8192 x 768 x 32768 (96 tiles, 192 workgroups) 405 / 390; more than 128 tiles
+// (5600 rows of 768 or 1024, 66 and 88 tiles, are refused too and would gain
+// 25% at 32768.)
 bool lm_head_dhidden_pays(int M, int N, int K) {
   const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-  if (tiles > 128) return false;
-  const int64_t by_cus = 256 / tiles;
-  return tiles * by_cus >= 205 || lm_head_dhidden_runs(M, N, K) < by_cus;
+  if (tiles > 128 || tiles * (256 / tiles) < 205) return false;
+  return (K + kGemmStep - 1) / kGemmStep >= (tiles <= 32 ? 63 : 94);
 }
 
 hipError_t launch_lm_head_dhidden(const void* g, int64_t ldg, const void* w, int64_t ldw, void* c, int64_t ldc, float* part,

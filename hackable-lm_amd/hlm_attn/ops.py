@@ -549,7 +549,8 @@ def lm_head_loss_impl(
     if stride * hidden.element_size() % 4096 == 0:
         stride += 64
     padded = hidden.new_empty((rows, stride))
-    padded[:, vocab:] = 0  # ce_dhidden_impl's contract; nothing writes there
+    if want_h and any(_lib.load().hlm_ce_dhidden_pays(r, hidden.shape[1], vocab) for r in {rows, n % rows}):
+        padded[:, vocab:] = 0  # hlm_ce_dhidden's contract; nothing writes there
     work = padded[:, :vocab]
     w_t = weight.t()
     for r0 in range(0, n, rows):

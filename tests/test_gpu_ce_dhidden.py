@@ -36,7 +36,12 @@ def test_rule_and_workspace():
     lib = _lib.load()
     pays, nbytes = lib.hlm_ce_dhidden_pays, lib.hlm_ce_dhidden_workspace_bytes
     assert pays(4096, 768, 32768) == 1 and nbytes(4096, 768, 32768) == 5 * 48 * 256 * 256 * 4
-    assert pays(904, 768, 50257) == 1 and pays(300, 256, 1000) == 1
+    assert pays(904, 768, 50257) == 1
+    # K has to be long, longer where there are more tiles, however few CUs the library's product takes
+    assert pays(272, 256, 3968) == 0 and pays(272, 256, 3969) == 1 and pays(300, 256, 1000) == 0
+    assert pays(8192, 256, 3969) == 1 and pays(8193, 256, 3969) == 0  # 32 tiles, 33
+    assert pays(4096, 2048, 5952) == 0 and pays(4096, 2048, 5953) == 1  # 128 tiles
+    assert pays(5600, 1024, 900) == 0 and pays(8192, 768, 600) == 0 and pays(8192, 768, 1000) == 0
     assert pays(8192, 768, 32768) == 0  # 96 tiles: two runs fill 192 CUs
     assert pays(16384, 768, 32768) == 0  # the chip is full without a split
     assert pays(4096, 772, 32768) == 0 and pays(0, 768, 32768) == 0  # not taken
@@ -127,7 +132,7 @@ def test_matches_the_product_of_the_same_operands(rows, hidden, vocab):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,hidden,vocab,stride", [(300, 256, 1000, 1024), (300, 260, 1000, 1024), (4096, 2304, 128, 128)])
+@pytest.mark.parametrize("rows,hidden,vocab,stride", [(300, 256, 1000, 1024), (300, 256, 4000, 4032), (300, 260, 1000, 1024), (4096, 2304, 128, 128)])
 def test_op_takes_either_product(rows, hidden, vocab, stride):
     """The op gives the same result where the kernel applies and where the
     library's product runs (hidden no multiple of 8; too many tiles)."""
