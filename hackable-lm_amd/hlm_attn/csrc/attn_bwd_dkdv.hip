@@ -448,16 +448,14 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_dkdv_merge_kernel(BwdArgs a
 // part by the number of chunks.  Fitted over 40 shapes, splitting pays while
 //   D = 64:  2 chunk + chunk blocks / 400 + blocks / 18 + 15 < 2 longest
 //   D = 128: 2 chunk + chunk blocks / 512 + blocks / 16 + 8 < 2 longest   (in query tiles of 32)
-// Up to 512 tokens and 52 query tiles D = 64 stays whole although it would gain
-// (333x4/1 W 129 32 -> 25): the tests hold the single-pass backward's dK and
-// dV to this path's bit for bit at such sizes.
 // Chunks that fill the slots one and a half or two times, or half, measured
 // slower (B = 2, T = 1777, 12 query on 4 kv heads, D = 128, causal: 20% at 1.5
 // and 2, 12% at 0.5).
 //
 // Whole backward (dQ in both as its own plan has it) with dK/dV unsplit ->
 // split (us), BxTxH/Hkv, causal unless W is given:
-//   taken    D = 64:  1500x4/4 47 -> 35, 1000x8/2 W 200 41 -> 29, 1024x12/12 39 -> 36, 2000x4/4 W 1024 42 -> 38
+//   taken    D = 64:  1500x4/4 47 -> 35, 1000x8/2 W 200 41 -> 29, 1024x12/12 39 -> 36, 2000x4/4 W 1024 42 -> 38,
+//                     333x4/1 W 129 32 -> 25, 512x8/4 34 -> 29, 2x400x8/2 W 300 46 -> 29, 128x16/2 30 -> 24
 //            D = 128: 2x1777x12/4 204 -> 110, 2000x4/4 W 1024 71 -> 55, 1024x16/16 61 -> 53, 1000x6/6 58 -> 49
 //   refused  D = 64:  2x2048x12/12 76 -> 78, 4096x16/16 153 -> 157, 2x1000x8/4 W 256 29 -> 30
 //            D = 128: 2048x16/16 W 512 48 -> 61, 4096x8/8 W 1024 74 -> 87, 500x8/8 the same
@@ -469,7 +467,6 @@ ChunkPlan dkdv_chunk_plan(int B, int T, int H, int Hkv, int D, int W) {
     return (std::min<int64_t>(T - 1, k0 + 126 + W) / 32 - k0 / 32 + 1) * G;
   };
   auto pays = [=](int64_t c, int64_t blocks, int64_t longest) {
-    if (D == 64 && T <= 512 && longest <= 52) return false;
     return (D == 64 ? 2 * c + c * blocks / 400 + blocks / 18 + 15 : 2 * c + c * blocks / 512 + blocks / 16 + 8) <
            2 * longest;
   };

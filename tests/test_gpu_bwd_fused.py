@@ -1,8 +1,8 @@
 """The single-pass backward (hlm_attn_bwd_fused, selected by HLM_ATTN_BWD=fused)
 against the two-kernel backward and the fp32 oracle (GPU only).
 
-dK and dV must equal the two-kernel path's bit for bit (same loop arithmetic,
-same workspace values); dQ, summed from bf16 partials of the 128-key tiles,
+dK and dV must equal the two-kernel path's (hlm_attn_bwd, which cuts no tile
+into chunks) bit for bit (same loop arithmetic, same workspace values); dQ, summed from bf16 partials of the 128-key tiles,
 must meet the gradient tolerances against the oracle (3e-2 norm-relative and
 elementwise, as in test_gpu_parity) and stay within 1e-2 norm-relative of
 the two-kernel dQ.
@@ -31,14 +31,24 @@ def _device() -> torch.device:
 def _both_backwards(q, k, v, do, window, dev, monkeypatch):
     """Forward once, then the two-kernel and the single-pass backward on the
     same device tensors; returns (two-kernel dq, dk, dv), (fused dq, dk, dv)."""
-    from hlm_attn import ops
+    from hlm_attn import _lib, ops
 
     qd, kd, vd, dod = (t.to(dev) for t in (q, k, v, do))
     w = 0 if window is None else window
     scale = 1.0 / math.sqrt(q.shape[-1])
     o, lse = ops.hip_attn_fwd(qd, kd, vd, w, scale)
     monkeypatch.delenv("HLM_ATTN_BWD", raising=False)
-    two = ops.hip_attn_bwd(dod, qd, kd, vd, o, lse, w, scale)
+    B, T, H, D = qd.shape
+    Hkv = kd.shape[2]
+    two = tuple(torch.empty_like(t) for t in (qd, kd, vd))
+    delta = torch.empty(2 * B * H * T, device=dev)
+    lib = _lib.load()
+    rc = lib.hlm_attn_bwd(*(t.data_ptr() for t in (qd, kd, vd, o, dod, lse, *two, delta)), B, T, H, Hkv, D,
+                          *(_lib.strides3(t) for t in (qd, kd, vd, o, dod, *two)), w, scale, ops._stream_handle(dev))
+    _lib.check(rc, lib)
+    default = ops.hip_attn_bwd(dod, qd, kd, vd, o, lse, w, scale)
+    if ops.bwd_split_bytes(B, T, H, Hkv, D, w) == 0:
+        assert all(torch.equal(a, b) for a, b in zip(two, default))
     monkeypatch.setenv("HLM_ATTN_BWD", "fused")
     assert ops.fused_backward_selected()
     fused = ops.hip_attn_bwd(dod, qd, kd, vd, o, lse, w, scale)

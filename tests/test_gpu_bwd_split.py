@@ -26,6 +26,8 @@ CASES = [
     (1, 1, 64, 1, 64, None),      # one token, one key tile, 64 query heads: chunks of whole heads
     (1, 1000, 8, 2, 64, 200),     # 44 query tiles a key tile
     (1, 129, 32, 1, 128, None),   # a second key tile of one row
+    (1, 333, 4, 1, 64, 129),      # few tokens, four heads to a key tile
+    (1, 128, 16, 2, 64, None),    # one key tile
     (1, 300, 40, 2, 64, 40),      # short window, many heads: chunks end inside a head
     (1, 777, 16, 1, 128, None),   # ragged, causal: key tiles with 1 to 16 chunks
     (2, 1025, 12, 4, 64, None),
@@ -64,7 +66,7 @@ def test_split_applies_to_the_cases_below(case):
         (8, 2048, 12, 12, 64, 512),    # the chip is full
         (1, 16384, 16, 16, 128, 2048),
         (1, 1000, 6, 6, 64, 300),      # short rows
-        (1, 333, 4, 1, 64, 129),
+        (1, 480, 6, 6, 64, None),
         (2, 1000, 8, 4, 64, 256),
         (1, 4096, 16, 16, 64, None),   # chunks would be as long as the slots they fill are slow
         (1, 4096, 8, 8, 128, 1024),
@@ -125,7 +127,7 @@ def test_split_backward_matches_the_unsplit_one_and_the_oracle(case):
         got.append((dq, dk, dv))
     one, two, again = got
     # By the sizes, the first cases cut dK/dV only and the others dQ or both.
-    assert torch.equal(one[0], two[0]) == (case in CASES[:7])
+    assert torch.equal(one[0], two[0]) == (case in CASES[:9])
     assert all(torch.equal(a, b) for a, b in zip(two, again)), "not deterministic"
     for name, a, b in zip(("dq", "dk", "dv"), one, two):
         a, b = a.float(), b.float()
