@@ -14,7 +14,7 @@
 //   caller (ops.eager_ext) uses them only where no tracing, dispatch mode,
 //   function transform or forward-mode AD is active; a backward that runs
 //   under one of these, or with create_graph, calls the custom op itself.
-#include <ATen/core/dispatch/Dispatcher.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
@@ -100,20 +100,26 @@ bool plain(const at::Tensor& t) {
 }
 
 // Whether a backward must go through its custom op: create_graph (the op then
-// refuses a second derivative), a dispatch mode, or a wrapped gradient.
+// refuses a second derivative), a dispatch or function mode, or a wrapped
+// gradient.
 bool needs_op(const variable_list& ts) {
-  if (at::GradMode::is_enabled() || c10::impl::TorchDispatchModeTLS::stack_len() > 0) return true;
+  if (at::GradMode::is_enabled() || c10::impl::TorchDispatchModeTLS::stack_len() > 0 ||
+      at::impl::PythonTorchFunctionTLS::stack_len() > 0)
+    return true;
   for (const auto& t : ts)
     if (!plain(t)) return true;
   return false;
 }
 
-// Calls hackable_lm::<name> through the dispatcher.
-variable_list call_op(const char* name, torch::jit::Stack stack) {
-  c10::Dispatcher::singleton().findSchemaOrThrow(name, "").callBoxed(stack);
-  variable_list out;
-  for (auto& v : stack) out.push_back(std::move(v).toTensor());
-  return out;
+// Calls torch.ops.hackable_lm.<name>, through Python: function modes see only
+// calls that are made there.
+template <class... Args>
+variable_list call_op(const char* name, Args&&... args) {
+  const py::gil_scoped_acquire gil;
+  const py::object op = py::module_::import("torch").attr("ops").attr("hackable_lm").attr(name).attr("default");
+  const py::object out = op(std::forward<Args>(args)...);
+  if (py::isinstance<py::tuple>(out)) return out.cast<variable_list>();
+  return {out.cast<at::Tensor>()};
 }
 
 void check(int rc) { TORCH_CHECK(rc == 0, "hip attention failed (code ", rc, "): ", hlm_attn_last_error()); }
@@ -153,7 +159,7 @@ struct Attention : torch::autograd::Function<Attention> {
     const at::Tensor none;
     if (needs_op({dout, s[0], s[1], s[2], s[3], s[4]}) || (s[0].size(3) == 64 && fused_backward_selected())) {
       const variable_list g =
-          call_op("hackable_lm::hip_attn_bwd", {dout, s[0], s[1], s[2], s[3], s[4], window, scale});
+          call_op("hip_attn_bwd", dout, s[0], s[1], s[2], s[3], s[4], window, scale);
       return {g[0], g[1], g[2], none, none};
     }
     const c10::Device dev = s[0].device();
@@ -222,8 +228,7 @@ struct QkNormRope : torch::autograd::Function<QkNormRope> {
     const double eps = ctx->saved_data["eps"].toDouble();
     const at::Tensor none;
     if (needs_op({grads[0], grads[1], saved[0], saved[1], saved[2], saved[3]})) {
-      const variable_list g = call_op("hackable_lm::hip_qk_norm_rope_backward",
-                                      {q, k, grads[0], grads[1], saved[2], saved[3], eps});
+      const variable_list g = call_op("hip_qk_norm_rope_backward", q, k, grads[0], grads[1], saved[2], saved[3], eps);
       return {g[0], g[1], none, none, none};
     }
     const c10::Device dev = q.device();
@@ -297,7 +302,7 @@ struct ResidualRmsNorm : torch::autograd::Function<ResidualRmsNorm> {
     const double eps = ctx->saved_data["eps"].toDouble();
     if (needs_op({grads[0], grads[1], saved})) {
       const variable_list g =
-          call_op("hackable_lm::hip_residual_rms_norm_backward", {saved, grads[0], grads[1], eps});
+          call_op("hip_residual_rms_norm_backward", saved, grads[0], grads[1], eps);
       return {g[0], g[0], at::Tensor()};
     }
     const c10::Device dev = saved.device();

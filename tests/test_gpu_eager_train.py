@@ -9,6 +9,7 @@ from __future__ import annotations
 import pytest
 import torch
 from torch.autograd import forward_ad
+from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 from torch.utils.checkpoint import checkpoint
 
@@ -225,6 +226,46 @@ def test_a_backward_under_a_dispatch_mode_shows_the_op(monkeypatch):
     fused = torch.autograd.grad(o, ins, do)
     assert torch.equal(fused[1], plain[1]) and torch.equal(fused[2], plain[2])
     assert ((fused[0].float() - plain[0].float()).norm() / plain[0].float().norm()).item() <= 1e-2
+
+
+class RecordFunctions(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.gpu
+def test_a_backward_under_a_function_mode_shows_the_op():
+    """torch.autograd.backward, which no function mode takes over, with the mode
+    active around it only."""
+    for make, name in ((_attn_inputs, "hip_attn_bwd"), (_producer_inputs, "hip_qk_norm_rope_backward"),
+                       (_residual_inputs, "hip_residual_rms_norm_backward")):
+        if make is _attn_inputs:
+            ins, do = make()
+            out, grads = [hlm_attn.attention(*ins, 50)], [do]
+        elif make is _producer_inputs:
+            ins, cos, sin = make()
+            out = hlm_attn.qk_norm_rope_hip(*ins, cos, sin, 1e-6)
+            grads = [t.detach() for t in out]
+        else:
+            ins = make()
+            out = hlm_attn.residual_rms_norm_hip(*ins, 1e-6)
+            grads = [t.detach() for t in out]
+        plain = torch.autograd.grad(out, ins, grads, retain_graph=True)
+        with RecordFunctions() as rec:
+            torch.autograd.backward(out, grads, retain_graph=True)
+        assert any(name in n for n in rec.names), rec.names
+        assert all(torch.equal(a, t.grad) for a, t in zip(plain, ins))
+    # an error inside the op arrives as it was raised
+    ins, do = _attn_inputs()
+    o = hlm_attn.attention(*ins, 50)
+    bad = torch.empty(do.numel() + 1, dtype=do.dtype, device=DEV)[1:].view(do.shape)
+    with RecordFunctions(), pytest.raises(RuntimeError, match="16-byte aligned"):
+        torch.autograd.backward([o], [bad])
 
 
 @pytest.mark.gpu
