@@ -138,3 +138,82 @@ def test_split_backward_matches_the_unsplit_one_and_the_oracle(case):
         rdq, rdk, rdv = oracle.backward(q, k, v, do, window)
         for name, a, r in zip(("dq", "dk", "dv"), two, (rdq, rdk, rdv)):
             assert_grad(name, a.float().cpu(), r)
+
+
+def _inputs(case, dev):
+    from hlm_attn import ops
+
+    B, T, H, Hkv, D, window = case
+    q, k, v, do = (t.to(dev) for t in make_inputs(B, T, H, Hkv, D, 70 + T))
+    w, scale = window or 0, 1.0 / math.sqrt(D)
+    o, lse = ops.hip_attn_fwd(q, k, v, w, scale)
+    return q, k, v, do, o, lse, w, scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[1], CASES[6], CASES[9], DQ_CASES[0], DQ_CASES[3], DQ_CASES[4]])
+def test_split_backward_reads_and_writes_any_strides(case):
+    """q, k, v as views of one projection, dO and o as (B, H, T, D), dq, dk and dv
+    into views of one gradient: bit-identical to contiguous tensors, and
+    nothing else in the buffers is written."""
+    from hlm_attn import ops
+
+    dev = torch.device("cuda", 0)
+    B, T, H, Hkv, D, _ = case
+    print(f"case split strides {case}", flush=True)
+    q, k, v, do, o, lse, w, scale = _inputs(case, dev)
+    want = ops.hip_attn_bwd(do, q, k, v, o, lse, w, scale)
+
+    def views(fill):
+        buf = torch.full((B, T, H + 2 * Hkv + 1, D), fill, dtype=torch.bfloat16, device=dev)
+        return buf, (buf[:, :, :H], buf[:, :, H : H + Hkv], buf[:, :, H + Hkv : -1])
+
+    _, ins = views(float("nan"))
+    for dst, src in zip(ins, (q, k, v)):
+        dst.copy_(src)
+    do_t, o_t = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (do, o))
+    gbuf, grads = views(7.0)
+    delta = torch.empty(2 * B * H * T, device=dev)
+    n = _bytes(*case)
+    part = torch.full((n // 4,), float("nan"), device=dev)
+    lib = _lib.load()
+    rc = lib.hlm_attn_bwd_split(*(t.data_ptr() for t in (*ins, o_t, do_t, lse, *grads, delta, part)), n, B, T, H, Hkv, D,
+                                *(_lib.strides3(t) for t in (*ins, o_t, do_t, *grads)), w, scale, ops._stream_handle(dev))
+    _lib.check(rc, lib)
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(grads, want))
+    assert bool((gbuf[:, :, -1] == 7).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [CASES[1], DQ_CASES[0], (1, 1500, 4, 2, 64, None)])
+def test_split_backward_in_a_graph(case):
+    """Forward and backward captured in a HIP graph, the workspace in its pool,
+    and replayed with eager work between: every replay equals the eager result."""
+    from hlm_attn import ops
+
+    dev = torch.device("cuda", 0)
+    print(f"case split graph {case}", flush=True)
+    q, k, v, do, _, _, w, scale = _inputs(case, dev)
+
+    def step():
+        o, lse = ops.hip_attn_fwd(q, k, v, w, scale)
+        return (o, lse, *ops.hip_attn_bwd(do, q, k, v, o, lse, w, scale))
+
+    eager = [t.clone() for t in step()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        static = step()
+    for replay in range(3):
+        for t in static:
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(static, eager)), f"replay {replay}"
+        step()  # the eager pool's workspace, of the same size
+        torch.cuda.synchronize()

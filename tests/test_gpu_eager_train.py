@@ -15,6 +15,7 @@ from torch.utils.checkpoint import checkpoint
 
 import hlm_attn
 from hlm_attn import ops
+from oracle import linear_ce as ce_oracle
 
 
 class Record(TorchDispatchMode):
@@ -150,6 +151,56 @@ def _side_stream():
     return (o, *g)
 
 
+def _chunked_inputs(D, T=1500):
+    """One sequence, full causal: dQ and dK/dV both run in chunks."""
+    g = torch.Generator().manual_seed(8)
+    ins = [torch.randn(1, T, h, D, generator=g).bfloat16().to(DEV).requires_grad_(True) for h in (4, 2, 2)]
+    assert ops.bwd_split_bytes(1, T, 4, 2, D, 0) > 0
+    return ins, torch.randn(1, T, 4, D, generator=g).bfloat16().to(DEV)
+
+
+def _chunked(D):
+    ins, do = _chunked_inputs(D)
+    o = hlm_attn.attention(*ins, None)
+    return (o, *torch.autograd.grad(o, ins, do))
+
+
+def _chunked_side_stream():
+    """The workspace is allocated and used on the backward's stream, with work
+    of another size on the main one meanwhile."""
+    ins, do = _chunked_inputs(64)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        o = hlm_attn.attention(*ins, None)
+        g = torch.autograd.grad(o, ins, do)
+    other = _chunked(128)
+    torch.cuda.current_stream().wait_stream(side)
+    for t in (o, *g):
+        t.record_stream(torch.cuda.current_stream())
+    return (o, *g, *other)
+
+
+def _lm_head(vocab):
+    """2500 tokens in chunks of 2048 and 452, ignored targets, against the float64
+    loss of the same bf16 values.  Roundings to bf16 (2^-9 of the value): of the
+    logits (below 4, so 2^-7 of a probability at most, 1e-3 of the loss), of
+    their gradient and of each product, twice for dW."""
+    g = torch.Generator().manual_seed(vocab)
+    hidden = torch.randn(2500, 128, generator=g).bfloat16()
+    weight = (torch.randn(vocab, 128, generator=g) * 0.05).bfloat16()
+    targets = torch.randint(0, vocab, (2500,), generator=g)
+    targets[::7] = -100
+    h, w = (t.to(DEV).requires_grad_(True) for t in (hidden, weight))
+    loss = hlm_attn.fused_linear_cross_entropy_with_weight(h, w, None, targets.to(DEV), chunk_size=2048)
+    grads = torch.autograd.grad(loss, (h, w))
+    ref_loss, *ref, _ = ce_oracle.fused_linear_cross_entropy(hidden, weight, None, targets, 2500)
+    assert abs(loss.item() - ref_loss.item()) <= 1e-3 * ref_loss.item()
+    for got, want in zip(grads, ref):
+        assert ((got.double().cpu() - want).norm() / want.norm()).item() <= 1e-2
+    return (loss.detach(), *grads)
+
+
 WAYS = {
     "attention": _attention,
     "attention_128": lambda: _attention(128, None),
@@ -164,6 +215,12 @@ WAYS = {
     "retained": _retained,
     "batched_gradient": _batched_gradient,
     "side_stream": _side_stream,
+    "chunked": lambda: _chunked(64),
+    "chunked_128": lambda: _chunked(128),
+    "chunked_side_stream": _chunked_side_stream,
+    "lm_head_odd": lambda: _lm_head(2049),       # rows padded to 2112 columns
+    "lm_head_4_kb_rows": lambda: _lm_head(2048), # 64 columns more
+    "lm_head_split": lambda: _lm_head(4097),     # dhidden with the vocabulary split
 }
 
 
