@@ -217,8 +217,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? 3 : 2) void attn_bwd_dkdv_kerne
   // address, lane part included, made opaque so it is not re-associated)
   // plus a constant that the ds_read offset field carries.  No address
   // arithmetic is left in the loop (24 VALU instructions per tile fewer at
-  // D = 64).  D = 128 has no registers to spare for them and recomputes
-  // the lane part, still with the slot constant folded.
+  // D = 64).  D = 128 has no registers to spare for them and forms each from
+  // ab0 or at00 by one XOR, still with the slot constant folded.
   static_assert(NBUF % 2 == 0, "a slot's parity is its tile's parity");
   unsigned ab_s[NS] = {}, atr[NDB][2] = {};
   if constexpr (KEEP_TRO) {

@@ -21,8 +21,8 @@
 // row's read as -inf, which neither the maximum nor the sum sees, and are not
 // written.  4096 rows of V = 50257 bf16 at a row stride of 50257: 529 us when
 // such rows were read three times, one element per lane; 169 us now (4.9 TB/s).  Rows
-// of more than 32 chunks per thread (V above 65528 bf16 or 32764 fp32) keep
-// that path.
+// of more than 32 chunks per thread (V above 65536 bf16 or 32768 fp32; rows
+// that are not aligned, above 65529 or 32765) keep that path.
 #include "attn_common.h"
 
 namespace hlm {

@@ -5,15 +5,16 @@
 //
 // K is the vocabulary, so C has few 256 x 256 tiles (48 for 4096 rows of 768)
 // and long sums; a product that gives each tile to one CU leaves most of the
-// chip idle (the library's: 322 us at K = 32768, 640 TFLOP/s).  Here S
+// chip idle (the library's: 320 us at K = 32768, 640 TFLOP/s).  Here S
 // workgroups share a tile, each summing a run of K, and a second kernel adds
-// their fp32 partial tiles in a fixed order: 176 us, 1170 TFLOP/s, 12 of them
-// the sum (K = 50257: 443 -> 263; 904 rows: 263 -> 115).  What bounds the
-// first kernel is its feed: 64 KB per CU and 64-deep step against 2048 cycles
-// of products.  With every step's tiles already in L2 it takes 40 us less.
+// their fp32 partial tiles in a fixed order.  Both kernels over fresh chunks of
+// G: 184-194 us, 1060-1120 TFLOP/s, 12 of them the sum (K = 50257: 450 -> 277-290;
+// 904 rows: 265 -> 118); inside the loss 193 + 12 us, the matrix cores 53% busy,
+// no bank conflicts, 390 MB read of 318.  What bounds the first kernel is its
+// feed: 64 KB per CU and 64-deep step against 2048 cycles of products.
 //
 // G's rows should not be a multiple of 4 KB apart: the 256 rows of a tile
-// then fall on few memory channels (217 us instead of 176).
+// then fall on few memory channels (220 us instead of 184).
 #include <algorithm>
 
 #include "attn_common.h"

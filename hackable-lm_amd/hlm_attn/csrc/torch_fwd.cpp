@@ -11,8 +11,8 @@
 //   differentiable calls of a training step as C++ autograd functions.  The
 //   Python custom ops that they stand for cost 70-170 us of host time per
 //   forward and backward, as much as or more than the kernels of a layer.  The
-//   caller (ops.eager_ext) uses them only where no tracing, dispatch mode,
-//   function transform or forward-mode AD is active; a backward that runs
+//   caller (ops.eager_ext) uses them only where no tracing, dispatch or function
+//   mode, function transform or forward-mode AD is active; a backward that runs
 //   under one of these, or with create_graph, calls the custom op itself.
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>

@@ -541,10 +541,10 @@ def lm_head_loss_impl(
     d_weight = weight.new_empty(weight.shape) if want_w else None
     d_bias = bias.new_zeros(bias.shape) if want_b else None
     losses = torch.empty(n, dtype=torch.float32, device=hidden.device)
-    # Rows of the workspace start on 128-byte lines: with V = 50257 the three
-    # products of a 4096-row chunk take 1132 us instead of 1275.
+    # Rows of the workspace start on 128-byte lines: with V = 50257 the
+    # library's three products of a 4096-row chunk take 1148 us instead of 1280.
     # They are not a multiple of 4 KB apart, which would put a column of them
-    # on few memory channels (dhidden 217 instead of 176 us at V = 32768).
+    # on few memory channels (dhidden 220 instead of 184 us at V = 32768).
     stride = -(-vocab // 64) * 64
     if stride * hidden.element_size() % 4096 == 0:
         stride += 64

@@ -264,8 +264,9 @@ int hlm_qk_norm_rope_bwd(const void* q, const void* k, const void* grad_q_out, c
  *                                                           the mean loss)
  * computed in fp32.  A target equal to ignore_index gives a zero loss and a
  * zero gradient row (F.cross_entropy's rule); any other target outside
- * [0, n_cols) gives NaN for that row.  Rows of up to 65528 bf16 or 32764 fp32
- * values, whatever their alignment, are read and written once.  Replaces the hackable_lm::linear_ce Triton op and its
+ * [0, n_cols) gives NaN for that row.  Rows of up to 65536 bf16 or 32768 fp32
+ * values (65529 or 32765 where a row begins or ends inside 16 bytes) are read
+ * and written once.  Replaces the hackable_lm::linear_ce Triton op and its
  * kernel (/root/reference/kernels.py:286-336) inside the chunked fused
  * linear cross-entropy (/root/reference/kernels.py:878-959).
  */
@@ -277,8 +278,8 @@ int hlm_ce_rows(void* logits, int logits_dtype, int64_t row_stride, const int64_
  * grad (n_rows x n_vocab, hlm_ce_rows' gradients), weight (n_vocab x
  * n_hidden) and dhidden (n_rows x n_hidden), rows at the given strides in
  * elements.  The columns n_vocab .. round_up(n_vocab, 64) - 1 of grad's rows
- * must exist and hold zeros.  n_hidden and the strides are multiples of 8, the
- * pointers 16-byte aligned.  Several workgroups share an output tile and their
+ * must exist and hold zeros (they are read).  n_hidden and the strides are
+ * multiples of 8, the pointers 16-byte aligned.  Several workgroups share an output tile and their
  * fp32 partial tiles, added in a fixed order, lie in ws: hlm_ce_dhidden_
  * workspace_bytes (0 possible), 16-byte aligned, no initialisation needed.
  * Stands where the reference calls its library product
