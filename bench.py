@@ -2,8 +2,8 @@
 """Benchmark of the HIP causal sliding-window attention backend on one MI355X.
 
 One "step" is one attention layer's forward + backward through the C ABI
-(hlm_attn_fwd, then hlm_attn_bwd on the forward's o and lse) at the BASELINE
-workload cfg2: B=8, H=12, T=2048, D=64, window=512, causal, bf16, synthetic
+(hlm_attn_fwd, then hlm_attn_bwd on the forward's o and lse) at the
+headline workload cfg2: B=8, H=12, T=2048, D=64, window=512, causal, bf16, synthetic
 N(0,1) inputs from one seed, resident in HBM before timing starts.  Warm
 cache: steps run back to back, as in training.
 
@@ -20,8 +20,8 @@ Prints ONE JSON line with, besides the contract fields: ms per layer (fwd,
 bwd, fwd+bwd), the fraction of MI355X's dense bf16 MFMA peak, per-kernel
 launch times, a roofline object for the dominant kernel (HIP-event mean over
 back-to-back launches), the CPU baseline (the reference's `torch` backend
-restated, configs[0] shape, fp32 forward, on the host's cores), and a
-"configs" object with every other BASELINE GPU config measured in the same
+restated, 2 x 1024 tokens, 6 heads, fp32 forward, on the host's cores), and a
+"configs" object with every other GPU workload measured in the same
 run: cfg3 (one full-causal layer), cfg4 (the 18-layer stack, per layer and in
 total) and cfg5 (q and k RoPE-rotated before the bf16 cast).  "producer",
 "eval", "lm_head" and "residual_norm" objects time the neighbouring kernels
@@ -63,7 +63,7 @@ CONFIGS = {
     "cfg4_full": dict(B=4, T=4096, H=12, D=128, W=None),
     "cfg5_long": dict(B=1, T=16384, H=16, D=128, W=2048),
 }
-CPU_CONFIG = dict(B=2, T=1024, H=6, D=64, W=256)
+CPU_CONFIG = dict(B=2, T=1024, H=6, D=64, W=256)  # the CPU baseline's workload
 KERNEL_NAMES = {"fwd": "attn_fwd_kernel", "bwd_dq": "attn_bwd_dq_kernel", "bwd_dkdv": "attn_bwd_dkdv_kernel"}
 
 
@@ -664,17 +664,17 @@ def measure_bwd_fused(names, reps: int, device, rounds: int = 5) -> dict:
 
 
 # ---------------------------------------------------------------------------
-# The other BASELINE configs, measured in the same run ("configs" object).
+# The other workloads, measured in the same run ("configs" object).
 # ---------------------------------------------------------------------------
 
-CFG4_LAYERS = dict(n_layer=18, window=1024, full_every=4)
-ROPE_BASE = 10000.0  # RoPE base 10000 over positions 0..T-1, whole head
+CFG4_LAYERS = dict(n_layer=18, window=1024, full_every=4)  # the 18-layer stack
+ROPE_BASE = 10000.0  # cfg5: RoPE base 10000 over positions 0..T-1, whole head
 
 
 def rope_rotate(x, base: float = ROPE_BASE):
     """Rotate-half RoPE over the whole head dim (model.py:105-114 with
     fraction 1.0, theta = base) of a (B, T, H, D) fp32 tensor, positions
-    0..T-1, computed in fp32: the input synthesis of BASELINE configs[4]."""
+    0..T-1, computed in fp32: the input synthesis of cfg5."""
     import torch
 
     T, D = x.shape[1], x.shape[3]
@@ -747,7 +747,7 @@ def measure_single_layer(name: str, reps: int, device, rope: bool = False, prewa
 
 
 def measure_layer_stack(passes: int, device, seed: int = 0) -> dict:
-    """18 attention layers (B=4, H=12, T=4096, D=128),
+    """cfg4: 18 attention layers (B=4, H=12, T=4096, D=128),
     layer l's window from the reference's pattern (layer_attention_window(l,
     18, 1024, 4): layers 3, 7, 11, 15 and 17 full causal) and its q, k, v, dO
     from seed + l.  One pass = the forwards of layers 0..17, then the
@@ -820,7 +820,7 @@ def measure_layer_stack(passes: int, device, seed: int = 0) -> dict:
 
 
 def measure_configs(device) -> dict:
-    """Every BASELINE GPU config besides the headline one, in this run."""
+    """Every GPU workload besides the headline one, in this run."""
     return {
         "data": "q, k, v, dO ~ N(0,1) from a seeded device generator (torch.Generator on the GPU), rounded to bf16; "
         "HIP-event means on the launch stream, warm cache",
@@ -847,13 +847,13 @@ def read_traffic(config: str, kernel: str):
 
 def cpu_baseline(budget_s: float = 10.0) -> dict:
     """The reference's `torch` backend (restated in oracle/, kernels.py:785-800)
-    on the host CPU: BASELINE configs[0], forward only, fp32."""
+    on the host CPU: CPU_CONFIG, forward only, fp32."""
     import torch
 
     from oracle import attention as oracle
 
     cfg = CPU_CONFIG
-    # As many threads as this process may run on (BASELINE.md's rule).
+    # As many threads as this process may run on.
     threads_before = torch.get_num_threads()
     cores = len(os.sched_getaffinity(0))
     torch.set_num_threads(cores)
@@ -905,7 +905,7 @@ def main() -> int:
     ap.add_argument("--warmup", type=int, default=20)
     ap.add_argument("--config", default="cfg2_local", choices=sorted(CONFIGS))
     ap.add_argument("--kernel-reps", type=int, default=500, help="back-to-back launches per kernel timing")
-    ap.add_argument("--no-configs", action="store_true", help="skip the other BASELINE configs (cfg3, cfg4, cfg5)")
+    ap.add_argument("--no-configs", action="store_true", help="skip the other workloads (cfg3, cfg4, cfg5)")
     ap.add_argument("--cold", action="store_true", help="also time per-launch medians with the cache flushed")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--graph", action="store_true", help="time HIP-graph replays of the step instead of eager launches")

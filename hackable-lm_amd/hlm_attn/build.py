@@ -3,7 +3,7 @@ CPython binding of its forward entry points (_pycall, host code, g++) and the
 torch C++ extension of plain eager calls (_torch_fwd, host code).
 
 Both are built in-tree next to this file, so they travel with the source tree
-to the GPU host.  Usage:  python -m hlm_attn.build  (or build()).
+to the machine that runs it.  Usage:  python -m hlm_attn.build  (or build()).
 """
 from __future__ import annotations
 

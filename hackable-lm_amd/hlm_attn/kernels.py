@@ -1,7 +1,7 @@
 """The hip branch of hackable-lm's attention dispatch.
 
 `scaled_dot_product_attention` keeps the signature of
-/root/reference/kernels.py:774-784 and behaves like its FlashAttention branch
+kernels.py:774-784 and behaves like its FlashAttention branch
 (kernels.py:816-841): an explicit mask is rejected, q/k/v are cast to bf16,
 the window becomes the kernels' causal look-back, the scale is 1/sqrt(D) and
 the result is bf16 in (B, T, H, D).  Like the FlashAttention-3/4 branches

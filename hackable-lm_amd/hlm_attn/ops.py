@@ -2,9 +2,9 @@
 
 They are registered the way the reference registers its Triton ops
 (torch.library.custom_op + register_fake + register_autograd,
-/root/reference/kernels.py:320,388,505 and :738-740), so a model that runs
+kernels.py:320,388,505 and :738-740), so a model that runs
 under torch.compile(fullgraph=True) and CUDA-graph capture
-(/root/reference/kernels.py:126-143) can trace and capture them: the fake
+(kernels.py:126-143) can trace and capture them: the fake
 implementations only describe shapes, and the real ones allocate through
 torch's caching allocator, launch on torch's current stream and never
 synchronise.  There is no CPU implementation: on a tensor that is not on a
@@ -313,7 +313,7 @@ hip_attn_fwd.register_autograd(_backward, setup_context=_setup_context)
 # --- the producer step: fused q/k RMSNorm + partial rotary embedding ---------------
 #
 # hackable_lm::hip_qk_norm_rope mirrors the reference's Triton op
-# hackable_lm::qk_norm_rope (/root/reference/kernels.py:505-535, autograd
+# hackable_lm::qk_norm_rope (kernels.py:505-535, autograd
 # :679-741): same inputs (q, k, cos, sin, eps), outputs contiguous in q's and
 # k's shapes, backward through the fused kernel.
 
@@ -442,7 +442,7 @@ hip_qk_norm_rope.register_autograd(_qk_backward, setup_context=_qk_setup_context
 # --- the LM head: cross-entropy rows of the fused linear + cross-entropy ----------
 #
 # hackable_lm::hip_linear_ce mirrors the reference's Triton op
-# hackable_lm::linear_ce (/root/reference/kernels.py:320-336): it overwrites
+# hackable_lm::linear_ce (kernels.py:320-336): it overwrites
 # `logits` in place with the gradient of the mean loss and returns the
 # per-row losses (already divided by n_tokens).
 
@@ -606,7 +606,7 @@ def _lm_head_loss_flops(hidden_shape, weight_shape, bias_shape, targets_shape, r
 # --- residual add + RMSNorm after the output / down projections -------------------
 #
 # hackable_lm::hip_residual_rms_norm computes residual_rms_norm
-# (/root/reference/model.py:73-75) on the GPU; the reference leaves its
+# (model.py:73-75) on the GPU; the reference leaves its
 # backward to autograd, here it is hackable_lm::hip_residual_rms_norm_backward.
 
 

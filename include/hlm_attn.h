@@ -5,8 +5,8 @@
  * This is the device boundary that hackable-lm's attention backends cross:
  * the reference calls `flash_attn_func(q, k, v, dropout_p, causal=True,
  * window_size=(W - 1, 0))` from `kernels.scaled_dot_product_attention`
- * (/root/reference/kernels.py:836-841), reached from
- * `AttentionCore.fwd_flash_attn_2` (/root/reference/model.py:216-226), and
+ * (kernels.py:836-841), reached from
+ * `AttentionCore.fwd_flash_attn_2` (model.py:216-226), and
  * autograd then runs FlashAttention-2's backward.  The two entry points below
  * replace that forward and that backward.
  *
@@ -66,8 +66,8 @@ int hlm_attn_abi_version(void);
  * Forward: o = softmax(scale * q k^T + mask) v, lse = logsumexp of the same
  * masked scores (natural log, fp32).
  * Replaces flash_attn_func(q, k, v, dropout_p=0.0, causal=True,
- * window_size=(window - 1, 0)) at /root/reference/kernels.py:841 and the
- * `torch` math at /root/reference/kernels.py:785-800.
+ * window_size=(window - 1, 0)) at kernels.py:841 and the
+ * `torch` math at kernels.py:785-800.
  */
 int hlm_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                  int B, int T, int H, int Hkv, int D,
@@ -110,8 +110,8 @@ int hlm_attn_fwd_split_count(int B, int T, int H, int D, int window);
  * -rowsum(dO * o), each as (B, H, T).  dk/dv are written completely (not
  * accumulated into).
  * Replaces the backward of flash_attn_func (FlashAttention-2's autograd
- * Function, called from /root/reference/kernels.py:841), i.e. the gradient
- * of the math at /root/reference/kernels.py:785-800.
+ * Function, called from kernels.py:841), i.e. the gradient
+ * of the math at kernels.py:785-800.
  */
 int hlm_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout,
                  const float* lse, void* dq, void* dk, void* dv, float* delta_ws,
@@ -180,7 +180,7 @@ int64_t hlm_attn_bwd_split_workspace_bytes(int B, int T, int H, int Hkv, int D, 
  * window) bytes, passed as partial_ws_bytes; other arguments as for
  * hlm_attn_bwd.  D != 64 returns HLM_ATTN_EUNSUPPORTED.  Replaces the same
  * call as hlm_attn_bwd (FlashAttention-2's backward behind
- * /root/reference/kernels.py:841); an alternative implementation of it,
+ * kernels.py:841); an alternative implementation of it,
  * selected by the caller.
  */
 int hlm_attn_bwd_fused(const void* q, const void* k, const void* v, const void* o, const void* dout,
@@ -234,8 +234,8 @@ int hlm_attn_bwd_noalloc(const void* q, const void* k, const void* v, const void
  * q_out / k_out are bf16 and contiguous.  D in {64, 128}; R a multiple of 16
  * with 0 <= R <= D; B * T * (H + Hkv) < 2^31 - 1024; eps > 0.
  * Replaces kernels.qk_norm_rope_triton / the hackable_lm::qk_norm_rope Triton
- * op (/root/reference/kernels.py:441-535, :756-771), the math of
- * QKVProjection.fwd_torch (/root/reference/model.py:101-115).
+ * op (kernels.py:441-535, :756-771), the math of
+ * QKVProjection.fwd_torch (model.py:101-115).
  */
 int hlm_qk_norm_rope_fwd(const void* q, const void* k, const void* cos, const void* sin, int table_dtype,
                          void* q_out, void* k_out, int B, int T, int H, int Hkv, int D, int rotary_dim,
@@ -247,8 +247,8 @@ int hlm_qk_norm_rope_fwd(const void* q, const void* k, const void* cos, const vo
  * (bf16, contiguous):  gn = the rotation transposed applied to grad_out,
  * grad_x = r (gn - z mean(gn z)), r = rsqrt(mean(x^2) + eps).
  * Replaces the hackable_lm::qk_norm_rope_backward Triton op
- * (/root/reference/kernels.py:541-665) and its CPU closed form
- * (/root/reference/kernels.py:703-741).
+ * (kernels.py:541-665) and its CPU closed form
+ * (kernels.py:703-741).
  */
 int hlm_qk_norm_rope_bwd(const void* q, const void* k, const void* grad_q_out, const void* grad_k_out,
                          const void* cos, const void* sin, int table_dtype, void* grad_q, void* grad_k,
@@ -267,8 +267,8 @@ int hlm_qk_norm_rope_bwd(const void* q, const void* k, const void* grad_q_out, c
  * [0, n_cols) gives NaN for that row.  Rows of up to 65536 bf16 or 32768 fp32
  * values (65529 or 32765 where a row begins or ends inside 16 bytes) are read
  * and written once.  Replaces the hackable_lm::linear_ce Triton op and its
- * kernel (/root/reference/kernels.py:286-336) inside the chunked fused
- * linear cross-entropy (/root/reference/kernels.py:878-959).
+ * kernel (kernels.py:286-336) inside the chunked fused
+ * linear cross-entropy (kernels.py:878-959).
  */
 int hlm_ce_rows(void* logits, int logits_dtype, int64_t row_stride, const int64_t* targets, float* loss, int n_rows,
                 int n_cols, int64_t n_tokens, int ignore_index, void* stream);
@@ -283,7 +283,7 @@ int hlm_ce_rows(void* logits, int logits_dtype, int64_t row_stride, const int64_
  * fp32 partial tiles, added in a fixed order, lie in ws: hlm_ce_dhidden_
  * workspace_bytes (0 possible), 16-byte aligned, no initialisation needed.
  * Stands where the reference calls its library product
- * (/root/reference/kernels.py:878-942).
+ * (kernels.py:878-942).
  */
 int hlm_ce_dhidden(const void* grad, int64_t grad_stride, const void* weight, int64_t weight_stride, void* dhidden,
                    int64_t dhidden_stride, int n_rows, int n_hidden, int n_vocab, void* ws, int64_t ws_bytes,
@@ -300,9 +300,9 @@ int hlm_ce_dhidden_pays(int n_rows, int n_hidden, int n_vocab);
  * n <= 8192)
  *   out    = residual + branch                  (bf16, as the bf16 add rounds it)
  *   normed = out * rsqrt(mean(out^2) + eps)     (fp32 from the rounded out, bf16)
- * Replaces residual_rms_norm (/root/reference/model.py:73-75) in
- * OutputProjection.fwd_torch (/root/reference/model.py:261-264) and
- * DownProjection.fwd_torch (/root/reference/model.py:303-304).
+ * Replaces residual_rms_norm (model.py:73-75) in
+ * OutputProjection.fwd_torch (model.py:261-264) and
+ * DownProjection.fwd_torch (model.py:303-304).
  */
 int hlm_residual_rms_norm_fwd(const void* residual, const void* branch, void* out, void* normed, int64_t rows, int n,
                               float eps, void* stream);

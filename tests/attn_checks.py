@@ -1,6 +1,6 @@
 """Size-independent checks of attention outputs over every (batch, head) slice.
 
-Used by the GPU parity tests at BASELINE's full sizes, where the exact oracle
+Used by the GPU parity tests at the full workload sizes, where the exact oracle
 covers only bands of a few slices; tests/test_invariants.py pins these checks
 on the CPU (they accept the oracle's bf16-rounded results and reject planted
 mistakes).  All three follow from the math of the `torch` backend

@@ -3,7 +3,7 @@ of holding Q pre-multiplied by scale * log2(e) in bf16, as the backward does.
 
 The backward may round Q * scale * log2(e) to bf16 because its outputs are
 checked at rel 3e-2.  The forward's logsumexp must stay within 1e-3 (the
-tolerance north_star states), and rounding the pre-scaled Q perturbs every
+tolerance that the parity tests hold it to), and rounding the pre-scaled Q perturbs every
 score by up to half a bf16 ulp of each Q element: on rows that see few keys
 the lse error then reaches several 1e-3.  Scaling the fp32 score instead (the
 kernel's fmaf(s, scale * log2(e), -m) before exp2) stays far inside 1e-3.
@@ -14,7 +14,7 @@ parity tests.  CPU only.
 """
 import numpy as np
 
-LSE_TOL = 1e-3  # north_star: logsumexp within 1e-3
+LSE_TOL = 1e-3  # the parity tests' bound on the logsumexp
 
 
 def _bf16(x):

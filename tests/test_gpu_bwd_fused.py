@@ -74,7 +74,7 @@ CASES = [
     (2, 200, 2, 2, 64, 3),
     (2, 300, 4, 2, 77, 5),       # grouped-query heads: one workgroup covers two query heads
     (1, 333, 4, 1, 129, 7),      # MQA, ragged, W not tile aligned
-    (2, 1024, 6, 6, 256, 8),     # BASELINE configs[0] shape
+    (2, 1024, 6, 6, 256, 8),     # the CPU baseline's shape
     (1, 700, 2, 2, None, 9),     # plain causal: up to 6 partials per row
     (1, 640, 2, 2, 513, 10),     # W = 4 * 128 + 1: the most partials per row for its window
 ]
@@ -95,7 +95,7 @@ def test_fused_backward_matches_oracle_and_two_kernel_path(B, T, H, Hkv, window,
 
 @pytest.mark.parametrize("name,B,T,H,window", [("cfg2", 8, 2048, 12, 512), ("cfg3", 8, 2048, 12, None)])
 def test_fused_backward_full_size(name, B, T, H, window, monkeypatch):
-    """BASELINE's D = 64 configs: the two paths agree (dK, dV exactly), and
+    """The D = 64 workloads: the two paths agree (dK, dV exactly), and
     the fused dQ of slice (b, h) = (0, 0) and (B - 1, H - 1) meets the
     oracle's tolerances."""
     dev = _device()

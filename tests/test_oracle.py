@@ -42,7 +42,7 @@ def test_layer_pattern_matches_reference_config_test():
     """tests/test_config.py:53-56 of the reference."""
     assert [oracle.layer_attention_window(i, 8, 512, 4) for i in range(8)] == [512, 512, 512, None, 512, 512, 512, None]
     assert [oracle.layer_attention_window(i, 3, 512, 4) for i in range(3)] == [512, 512, None]
-    # BASELINE cfg4: 18 layers, W=1024, every 4th full, plus the last layer.
+    # cfg4: 18 layers, W=1024, every 4th full, plus the last layer.
     pattern = [oracle.layer_attention_window(i, 18, 1024, 4) for i in range(18)]
     assert [i for i, w in enumerate(pattern) if w is None] == [3, 7, 11, 15, 17]
     assert oracle.layer_attention_window(0, 4, None, 4) is None
