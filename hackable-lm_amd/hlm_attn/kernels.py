@@ -311,6 +311,9 @@ def fused_linear_cross_entropy_with_weight(
     targets_flat = targets.reshape(-1).contiguous()
     if hidden_flat.device.type != "cuda":
         raise RuntimeError("the hip fused linear cross entropy runs on ROCm devices only")
+    if not torch.is_grad_enabled():  # which the autograd function does not see: it would form the gradients
+        hidden_flat, weight = hidden_flat.detach(), weight.detach()
+        bias = None if bias is None else bias.detach()
     return _LMHeadLoss.apply(hidden_flat, weight, targets_flat, bias, chunk_size)
 
 

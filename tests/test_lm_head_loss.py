@@ -98,6 +98,26 @@ def test_loss_traces_with_fullgraph_as_one_op(vocab, with_bias):
     assert [c for c in calls if "hackable_lm" in c] == ["hackable_lm.hip_lm_head_loss.default"], calls
 
 
+@pytest.mark.parametrize("grad", [True, False])
+def test_a_traced_loss_forms_no_gradients_without_grad_mode(grad):
+    """The op's products cannot be dropped from a graph as dead code, so a
+    compiled no-grad loss (an evaluation) must not ask for them, whatever its
+    inputs require."""
+    flags = []
+
+    def backend(gm, example_inputs):
+        flags.extend(n.args[-3:] for m in gm.modules() if isinstance(m, torch.fx.GraphModule)
+                     for n in m.graph.nodes if "hip_lm_head_loss" in str(n.target))
+        return gm.forward
+
+    torch._dynamo.reset()
+    with FakeTensorMode(allow_non_fake_inputs=True), torch.set_grad_enabled(grad):
+        h, w, b = (torch.empty(s, dtype=torch.bfloat16, device="cuda", requires_grad=True) for s in ((96, 64), (1000, 64), (1000,)))
+        targets = torch.empty(96, dtype=torch.int64, device="cuda")
+        torch.compile(hlm_attn.fused_linear_cross_entropy_with_weight, fullgraph=True, backend=backend)(h, w, b, targets)
+    assert flags == [(grad, grad, grad)]
+
+
 @pytest.mark.parametrize("wanted,products", [((), 1), ((0,), 2), ((0, 1, 2), 3)])
 def test_the_op_and_the_direct_loop_agree(cpu_rows, wanted, products):
     """A dispatch mode sees the op, with the FLOPs of its products."""
